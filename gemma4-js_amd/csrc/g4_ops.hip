@@ -968,18 +968,21 @@ __global__ __launch_bounds__(kBlock) void attn_dec_kernel(const float *__restric
 // Merges split partials:
 //   out = sum_s e^(m_s - M) o_s / sum_s e^(m_s - M) l_s.
 // Block (query row, head, 64-dim slice).  Each thread issues the loads of the
-// first 16 of its splits (s = wave + 4 i) before anything else; the 4 waves'
-// sums meet in LDS.  Splits beyond the keys of this call (kpw > 0:
+// first 16 of its splits (s = wave + NW i) before anything else; the waves'
+// sums meet in LDS.  Bound by those loads' latency: 16 waves where 4 would
+// walk past 16 splits each (one row over 3001 keys, head dim 512, 188 splits:
+// combine 21.9 -> 7.5 us, the call 30.7 -> 15.4).  Splits beyond the keys of this call (kpw > 0:
 // ceil(keylen / kpw) splits) were not written.
-__global__ __launch_bounds__(kBlock) void attn_combine_kernel(const float *__restrict__ part,
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void attn_combine_kernel(const float *__restrict__ part,
                                                               int H, int hd, int kpw,
                                                               int nsplit, int keylen,
                                                               const int *__restrict__ pos_dev,
                                                               int qrows, float *__restrict__ out) {
   constexpr int U = 16;
-  __shared__ float red[4];
-  __shared__ float accs[4][64];
-  __shared__ float ls4[4];
+  __shared__ float red[NW];
+  __shared__ float accs[NW][64];
+  __shared__ float lsw[NW];
   const int dslices = hd >> 6;
   const int b = blockIdx.x;
   const int dsl = b % dslices, qh = b / dslices;
@@ -994,23 +997,26 @@ __global__ __launch_bounds__(kBlock) void attn_combine_kernel(const float *__res
   float mv[U], lv[U], ov[U];
 #pragma unroll
   for (int i = 0; i < U; ++i) {
-    const int sp = wave + 4 * i;
+    const int sp = wave + NW * i;
     const float *ps = pb + (size_t)(sp < ns ? sp : 0) * sstep;  // clamped: no branch
     const float m0 = ps[0], l0 = ps[1], o0 = ps[2 + d];
     mv[i] = sp < ns ? m0 : -3.4e38f;
     lv[i] = sp < ns ? l0 : 0.f;
     ov[i] = sp < ns ? o0 : 0.f;
   }
-  // block max of all split maxima (splits past 4U are read again below)
+  // block max of all split maxima (splits past NW U are read again below)
   float mx = -3.4e38f;
 #pragma unroll
   for (int i = 0; i < U; ++i) mx = fmaxf(mx, mv[i]);
-  for (int sp = wave + 4 * U; sp < ns; sp += 4) mx = fmaxf(mx, pb[(size_t)sp * sstep]);
+#pragma unroll 4
+  for (int sp = wave + NW * U; sp < ns; sp += NW) mx = fmaxf(mx, pb[(size_t)sp * sstep]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
   if (lane == 0) red[wave] = mx;
   __syncthreads();
-  const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float M = red[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) M = fmaxf(M, red[i]);
   float acc = 0.f, lsum = 0.f;
 #pragma unroll
   for (int i = 0; i < U; ++i) {
@@ -1018,19 +1024,24 @@ __global__ __launch_bounds__(kBlock) void attn_combine_kernel(const float *__res
     acc = fmaf(w, ov[i], acc);
     lsum = fmaf(w, lv[i], lsum);
   }
-  for (int sp = wave + 4 * U; sp < ns; sp += 4) {
+#pragma unroll 4
+  for (int sp = wave + NW * U; sp < ns; sp += NW) {
     const float *ps = pb + (size_t)sp * sstep;
     const float w = expf(ps[0] - M);
     acc = fmaf(w, ps[2 + d], acc);
     lsum = fmaf(w, ps[1], lsum);
   }
   accs[wave][lane] = acc;
-  if (lane == 0) ls4[wave] = lsum;
+  if (lane == 0) lsw[wave] = lsum;
   __syncthreads();
   if (wave == 0) {
-    const float L = ls4[0] + ls4[1] + ls4[2] + ls4[3];
-    out[((size_t)qr * H + h) * hd + d] =
-        (accs[0][lane] + accs[1][lane] + accs[2][lane] + accs[3][lane]) / L;
+    float L = lsw[0], sum = accs[0][lane];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) {
+      L += lsw[i];
+      sum += accs[i][lane];
+    }
+    out[((size_t)qr * H + h) * hd + d] = sum / L;
   }
 }
 
@@ -1237,6 +1248,20 @@ size_t attention_part_floats(int qrows, int heads, int hd, int max_keylen, int k
   return (multi > single ? multi : single) * heads * ((size_t)hd + 2);
 }
 
+// 4 waves per block hold up to 64 splits in one round of loads, 16 waves 256.
+int launch_combine(const float *part, int heads, int hd, int kpw, int nsplit, int keylen,
+                   const int *pos_dev, int qrows, float *out) {
+  const dim3 grid(qrows * heads * (hd / 64));
+  if (nsplit > 64)
+    hipLaunchKernelGGL(attn_combine_kernel<16>, grid, dim3(1024), 0, stream(), part, heads, hd, kpw,
+                       nsplit, keylen, pos_dev, qrows, out);
+  else
+    hipLaunchKernelGGL(attn_combine_kernel<4>, grid, dim3(256), 0, stream(), part, heads, hd, kpw,
+                       nsplit, keylen, pos_dev, qrows, out);
+  G4_LAUNCH_CHECK("attn_combine_kernel");
+  return G4_OK;
+}
+
 int launch_attention(const float *q, const float *k, const float *v, int qrows, int heads,
                      int hd, int keylen, int qpos0, const int *pos_dev, int max_keylen,
                      bool sliding, int window, int kpw, float *part, float *out, void *xt,
@@ -1259,10 +1284,7 @@ int launch_attention(const float *q, const float *k, const float *v, int qrows, 
       default: return fail(G4_E_ARG, "attention: head_dim %d must be 64, 128, 256 or 512", hd);
     }
     G4_LAUNCH_CHECK("attn_dec_kernel");
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(heads * (hd / 64)), dim3(kBlock), 0, stream(),
-                       part, heads, hd, 0, ns, keylen, pos_dev, qrows, out);
-    G4_LAUNCH_CHECK("attn_combine_kernel");
-    return G4_OK;
+    return launch_combine(part, heads, hd, 0, ns, keylen, pos_dev, qrows, out);
   }
   kpw = split_kpw(kpw, max_keylen);
   AttnArgs a;
@@ -1316,10 +1338,7 @@ int launch_attention(const float *q, const float *k, const float *v, int qrows, 
     default: return fail(G4_E_ARG, "attention: head_dim %d must be 64, 128, 256 or 512", hd);
   }
   G4_LAUNCH_CHECK("attn_split_kernel");
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(qrows * heads * (hd / 64)), dim3(kBlock), 0,
-                     stream(), part, heads, hd, kpw, a.nsplit, keylen, pos_dev, qrows, out);
-  G4_LAUNCH_CHECK("attn_combine_kernel");
-  return G4_OK;
+  return launch_combine(part, heads, hd, kpw, a.nsplit, keylen, pos_dev, qrows, out);
 }
 
 int launch_ple_mix(const float *proj, float pre_scale, const float *norm_scale,

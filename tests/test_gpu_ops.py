@@ -224,6 +224,21 @@ def test_attention_rows_cache_longer_than_keylen(g4, qrows):
     check_attention(got, want, fp32_attention(q, k, v, qrows, heads, hd, keylen, qpos0, True, 16))
 
 
+# One row's key splits: 64 and fewer, more, and more than one round of loads holds.
+@pytest.mark.parametrize("hd,keylen", [(256, 1024), (256, 1040), (512, 4097), (64, 6000)])
+def test_attention_one_row_many_splits(g4, hd, keylen):
+    rng = np.random.default_rng([hd, keylen])
+    q = rng.standard_normal((1, 8 * hd)).astype(np.float32) * np.float32(hd ** -0.25)
+    k = rng.standard_normal((keylen, hd)).astype(np.float32) * np.float32(hd ** -0.25)
+    v = rng.standard_normal((keylen, hd)).astype(np.float32)
+    qpos0 = keylen - 1
+    y = out(g4, 8 * hd)
+    g4.attention(dev(g4, q), dev(g4, k), dev(g4, v), 1, 8, hd, keylen, qpos0, False, 0, y)
+    got = y.download(np.float32).reshape(1, 8 * hd)
+    want = lo.attention(q, k, v, 1, 8, hd, keylen, qpos0, False, 0)
+    check_attention(got, want, fp32_attention(q, k, v, 1, 8, hd, keylen, qpos0, False, 0))
+
+
 def test_ple_mix(g4):
     rng = np.random.default_rng(12)
     rows, width, layers = 4, 256, 35
