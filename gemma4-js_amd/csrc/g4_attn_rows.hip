@@ -1,0 +1,895 @@
+// Attention of many query rows over the FP32 KV cache (QK_SHADER,
+// SOFTMAX_SHADER and ATTN_OUT_SHADER, gpu-runtime.js:1204-1248) on the 16-bit
+// matrix cores.
+//
+// Numerics.  The 16-bit matrix forms run at 16 times the FP32 form's rate, so
+// FP32 operands are split and the sums stay in FP32.
+//   scores   q and k as three BF16 parts each (exact: 3 x 8 bits), six
+//            v_mfma_f32_16x16x32_bf16; the dropped products are below 2^-26.
+//            An error of a score is a relative error of its probability, and
+//            two FP16 parts (22 bits, three products) left 1.3-1.7 times the
+//            FP32 form's error at head dim 512.
+//   outputs  v and p as two FP16 parts 2^e (hi + lo), three
+//            v_mfma_f32_16x16x32_f16 (hi.hi, hi.lo, lo.hi).  v has one
+//            exponent per key, folded into that key's probability; p has one
+//            per query row and key tile (that of the tile's largest p 2^e_v),
+//            so no range of values is out of reach.
+//
+// Two launches, three where the keys are split over blocks:
+//   attn_kv_split_kernel    k and v of the visible keys as FP16 hi/lo in the
+//                           order the matrix instructions read them
+//   attn_rows_f16_kernel    64 rows of [qrows * heads, hd] per block
+//   attn_rows_merge_kernel  adds the key splits
+//
+// Measured (us per call, 8 heads, against the FP32 matrix kernels in
+// g4_ops.hip on one box; error against binary64 in parentheses):
+//   head dim 512, all keys   2048 rows, 4096 keys   1387 (8.0e-7) -> 622 (4.1e-7)
+//                            1500 rows, 3000 keys    785 (7.1e-7) -> 464 (3.8e-7)
+//                            20 rows, 2020 keys      216 -> 40
+//                            512 rows, 512 keys       61 (3.0e-7) -> 49 (2.3e-7)
+//   head dim 256, window 512 1500 rows, 3000 keys    103 (4.8e-7) -> 70 (3.0e-7)
+//                            20 rows, 2020 keys       35 -> 24
+// The long case is 170 TFLOP/s in FP32 terms.  Its block step of 32 keys takes
+// about 5 us against 2 us of matrix work: with the loads left out it was 70% of
+// the time, with the score products left out 59%, with softmax and barriers
+// alone 30%.
+#include <math.h>
+
+#include <type_traits>
+
+#include "g4_gemv.h"
+#include "g4_internal.h"
+#include "g4_ops.h"
+
+namespace g4 {
+
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kTile = 32;      // keys per tile
+constexpr int kRows = 64;      // query rows (of qrows * heads) per block
+constexpr int kMaxSplits = 64;  // key splits of one call
+// Per tile: [0, 32) 2^(e_v - max e_v) of each key, 32 max e_v, 33 and 34 the
+// flags of K and V.
+constexpr int kMetaInts = 64;
+
+struct RowsArgs {
+  const float *q, *k, *v;
+  float *out;
+  uint4 *xt;  // the prefill GEMM's x' (w4_gemm_prepare), instead of out
+  int *xe;
+  int Mp;
+  u32x4 *kv;   // split tiles: 32 hd 6 bytes of K, then 32 hd 4 of V
+  int *meta;   // per tile kMetaInts
+  float *part;  // [splits][nrows][hd] unnormalised outputs
+  float2 *ml;   // [splits][nrows] (max, sum)
+  int H, hd, keylen, qpos0, sliding, window, qrows;
+  int tps;  // key tiles per split
+  const int *pos_dev;
+};
+
+// Positions and key tiles of a call or of one block's rows.
+struct Span {
+  int qpos0, keylen, nrows;
+  __device__ explicit Span(const RowsArgs &a) {
+    qpos0 = a.pos_dev ? *a.pos_dev : a.qpos0;
+    keylen = a.pos_dev ? qpos0 + a.qrows : a.keylen;
+    nrows = a.qrows * a.H;
+  }
+  __device__ int kmin(const RowsArgs &a, int pos) const {
+    const int lo = a.sliding ? pos - a.window + 1 : 0;
+    return lo > 0 ? lo : 0;
+  }
+  // first tile of the call: the tile slots count from it
+  __device__ int base(const RowsArgs &a) const { return kmin(a, qpos0) / kTile; }
+  __device__ int kmax(int pos) const { return pos < keylen - 1 ? pos : keylen - 1; }
+};
+
+__device__ __forceinline__ uint32_t pack_h2(_Float16 a, _Float16 b) {
+  return __builtin_bit_cast(uint32_t, (f16x2){a, b});
+}
+
+// 8 values as three BF16 parts, each the rounding of what the ones before
+// leave (differences of FP32 values that are exact).
+__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[3]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    p[0][i] = (__bf16)x[i];
+    const float r = x[i] - (float)p[0][i];
+    p[1][i] = (__bf16)r;
+    p[2][i] = (__bf16)(r - (float)p[1][i]);
+  }
+}
+
+// Exponent that brings a row of largest magnitude mx (as bits) to [2^13, 2^14).
+__device__ __forceinline__ int row_exp(uint32_t mx) {
+  return __builtin_amdgcn_frexp_expf(__uint_as_float(mx)) - 14;
+}
+
+// max over the lanes c, c + 16, c + 32, c + 48
+__device__ __forceinline__ float group_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr uint32_t kInfBits = 0x7f800000u;
+constexpr uint32_t kBf16MaxBits = 0x7f7f8000u;  // from here on BF16 rounds to infinity
+constexpr int kZeroExp = -200;  // e_v of an all-zero row: its probability becomes 0
+
+// Waves that share a row's head dim (its q and output dims), and the place of
+// V piece n: first the first halves of every such wave's dims.
+template <int HD>
+constexpr int kDimWaves = HD > 256 ? 2 : 1;
+template <int HD>
+__device__ constexpr int v_piece(int n) {
+  constexpr int NN = HD / 16, NW = NN / kDimWaves<HD>;
+  const int dh = n / NW, i = n % NW;
+  return (i / (NW / 2)) * (NN / 2) + dh * (NW / 2) + i % (NW / 2);
+}
+
+// K (blockIdx.y 0) or V (1) of one 32-key tile.  K piece (sub, j) is the A
+// operand of score step j for keys 16 sub ..: lane (c, g) holds key c, dims
+// 32 j + 8 g .. + 7, three parts of 1 KB.  V piece n is the A operand of output
+// dims 16 n ..: lane (c, g) holds dim 16 n + c of keys 4 g .. + 3 and 16 + 4 g
+// .. + 3, the keys whose probabilities lane group g computes, 1 KB of hi and
+// 1 KB of lo.  Rows past the last visible key are zeros and are not read.  A
+// row with a non-finite value is stored as zeros and flags its tile, which
+// the attention kernel then computes from the FP32 rows.  Bound by the
+// latency of its loads and of the reduction behind them.
+template <int HD>
+__global__ __launch_bounds__(512) void attn_kv_split_kernel(RowsArgs a) {
+  constexpr int KI = (HD / 32 + 3) / 4, VI = (HD / 16 + 7) / 8;
+  __shared__ uint32_t mxs[8][32];
+  __shared__ int flag;
+  const Span sp(a);
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, c = lane & 15, g = lane >> 4;
+  const int slot = blockIdx.x, k0 = (sp.base(a) + slot) * kTile;
+  const int kmax = sp.kmax(sp.qpos0 + a.qrows - 1);
+  if (k0 > kmax) return;
+  u32x4 *dst = a.kv + (size_t)slot * (20 * HD) + (blockIdx.y ? 12 * HD : 0);
+  int *meta = a.meta + (size_t)slot * kMetaInts;
+  if (t == 0) flag = 0;
+  if (blockIdx.y == 0) {
+    const int sub = w & 1, key = k0 + 16 * sub + c;
+    const float *src = a.k + (size_t)(key <= kmax ? key : kmax) * HD + 8 * g;
+    float x[KI][8];
+    uint32_t mx = 0;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const int j = (w >> 1) + 4 * i;
+      const float4 *p = reinterpret_cast<const float4 *>(src + 32 * (j < HD / 32 ? j : 0));
+      const float4 u0 = p[0], u1 = p[1];
+      const float y[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        x[i][e] = key <= kmax ? y[e] : 0.f;
+        const uint32_t b = __float_as_uint(x[i][e]) & 0x7fffffffu;
+        mx = b > mx ? b : mx;
+      }
+    }
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1) {
+      const uint32_t b = __shfl_xor(mx, o, 64);
+      mx = b > mx ? b : mx;
+    }
+    if (g == 0) mxs[w][c] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t b = mxs[2 * i + sub][c];
+      mx = b > mx ? b : mx;
+    }
+    const bool bad = mx >= kBf16MaxBits;
+    if (bad) flag = 1;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const int j = (w >> 1) + 4 * i;
+      if (j >= HD / 32) continue;
+      if (bad)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[i][q] = 0.f;
+      bf16x8 p[3];
+      split8(x[i], p);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        dst[((sub * (HD / 32) + j) * 3 + q) * 64 + lane] = __builtin_bit_cast(u32x4, p[q]);
+    }
+    __syncthreads();
+    if (t == 0) meta[33] = flag;
+  } else {
+    float x[VI][8];
+    uint32_t mx[8] = {};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int key = k0 + (e < 4 ? 4 * g + e : 12 + 4 * g + e);
+      const float *src = a.v + (size_t)(key <= kmax ? key : kmax) * HD + c;
+#pragma unroll
+      for (int i = 0; i < VI; ++i) {
+        const int n = w + 8 * i;
+        const float y = src[16 * (n < HD / 16 ? n : 0)];
+        x[i][e] = key <= kmax ? y : 0.f;
+        const uint32_t b = __float_as_uint(x[i][e]) & 0x7fffffffu;
+        mx[e] = b > mx[e] ? b : mx[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+      for (int o = 1; o <= 8; o <<= 1) {
+        const uint32_t b = __shfl_xor(mx[e], o, 64);
+        mx[e] = b > mx[e] ? b : mx[e];
+      }
+      if (c == 0) mxs[w][8 * g + e] = mx[e];
+    }
+    __syncthreads();
+    int ev[8];
+    bool bad[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      uint32_t m = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t b = mxs[i][8 * g + e];
+        m = b > m ? b : m;
+      }
+      bad[e] = m >= kInfBits;
+      ev[e] = bad[e] || m == 0 ? kZeroExp : row_exp(m);
+      if (bad[e]) flag = 1;
+    }
+    int em = ev[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) em = ev[e] > em ? ev[e] : em;
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1) {
+      const int b = __shfl_xor(em, o, 64);
+      em = b > em ? b : em;
+    }
+    if (w == 0 && c == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        meta[e < 4 ? 4 * g + e : 12 + 4 * g + e] = __float_as_int(ldexpf(1.f, ev[e] - em));
+      if (g == 0) meta[32] = em;
+    }
+#pragma unroll
+    for (int i = 0; i < VI; ++i) {
+      const int n = w + 8 * i;
+      if (n >= HD / 16) continue;
+      f16x8 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float s = bad[e] ? 0.f : ldexpf(x[i][e], -ev[e]);
+        hi[e] = (_Float16)s;
+        lo[e] = (_Float16)(s - (float)hi[e]);
+      }
+      const int at = v_piece<HD>(n);
+      dst[(2 * at) * 64 + lane] = __builtin_bit_cast(u32x4, hi);
+      dst[(2 * at + 1) * 64 + lane] = __builtin_bit_cast(u32x4, lo);
+    }
+    __syncthreads();
+    if (t == 0) meta[34] = flag;
+  }
+}
+
+// One row's 8-value chunk halves as the prefill GEMM's x' (pair order (0,4)
+// (1,5) (2,6) (3,7), hi plane and lo plane): the even lane group of a pair
+// holds values 0-3 and writes the hi chunk, the odd one holds 4-7 and writes
+// the lo chunk.
+__device__ __forceinline__ u32x4 xprep_chunk(const float (&v)[4], int e, bool odd) {
+  _Float16 h[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float s = ldexpf(v[i], -e);
+    h[i] = (_Float16)s;
+    l[i] = (_Float16)(s - (float)h[i]);
+  }
+  const uint32_t h01 = pack_h2(h[0], h[1]), h23 = pack_h2(h[2], h[3]);
+  const uint32_t l01 = pack_h2(l[0], l[1]), l23 = pack_h2(l[2], l[3]);
+  const uint32_t r01 = __shfl_xor(odd ? h01 : l01, 16, 64);
+  const uint32_t r23 = __shfl_xor(odd ? h23 : l23, 16, 64);
+  const uint32_t a01 = odd ? r01 : h01, a23 = odd ? r23 : h23;  // values 0-3
+  const uint32_t b01 = odd ? l01 : r01, b23 = odd ? l23 : r23;  // values 4-7
+  return (u32x4){(a01 & 0xffffu) | (b01 << 16), (a01 >> 16) | (b01 & 0xffff0000u),
+                 (a23 & 0xffffu) | (b23 << 16), (a23 >> 16) | (b23 & 0xffff0000u)};
+}
+
+// A block owns 64 rows of [qrows * heads, hd] (row R at position qpos0 +
+// R / H, seeing the keys (pos - window, pos] or [0, pos]), 16 per wave (head
+// dim 512: per two waves with half of the dims each, which add their scores
+// through LDS, so that two waves' registers fit a SIMD), and key tiles blockIdx.y tps .. of its rows' range.  Lane (c, g) of a wave
+// works for row c throughout:
+//   S^T = K . Q^T   lane (c, g) gets keys 4 g .. + 3 and 16 + 4 g .. + 3
+//   softmax         a lane's 8 scores, then lane groups by two exchanges
+//   O^T += V^T . P^T  the lane's probabilities are its operand as they are,
+//                   so P never leaves the registers
+// Tiles reach LDS by direct loads, in three buffers: A the K of keys 0-15, B
+// that of keys 16-31 and then the second half of V's dims, C the first half.
+//   S0 (A) | S1 (B), softmax, O0 (C) | ... O1 (B)
+// A's next load leaves after S0, B's after S1 (V) and after O1 (K), C's after
+// O0, so each load has at least one phase to land in: one wait and barrier
+// per phase.  At head dim 512 whole K and V tiles beside each other would not
+// fit 160 KB; at 256 two blocks fit a CU.
+// Masked keys get weight exactly 0; tiles that a wave's rows do not see are
+// skipped by that wave.
+template <int HD>
+__global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(RowsArgs a) {
+  constexpr int DH = kDimWaves<HD>, WV = 4 * DH, NTH = 64 * WV;
+  constexpr int NJ = HD / 32 / DH, NN = HD / 16 / DH;  // of one wave's dims
+  constexpr int KP = 3 * NJ * DH, VP = NN * DH;        // 1 KB pieces of 16 keys of K, of V's half
+  constexpr int KW = (KP + WV - 1) / WV, VW = VP / WV;  // and loads per wave
+  constexpr int KU = KP * 64, VU = VP * 64;             // units of a buffer
+  struct Smem {
+    u32x4 a[KU];
+    u32x4 b[KU > VU ? KU : VU];
+    u32x4 c[VU];
+    int meta[kMetaInts];
+    f32x4 ex[DH > 1 ? WV : 0][2][64];  // partial scores of waves that share rows
+    float mx[DH > 1 ? WV : 0][16];
+  };
+  __shared__ Smem sm;
+  typedef __attribute__((address_space(3))) void *lds_ptr;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int rg = w & 3, dh = w >> 2;  // rows 16 rg .., dims dh HD / DH ..
+  const Span sp(a);
+  const int H = a.H, nrows = sp.nrows;
+  // the last rows see the most keys: they start first
+  const int R0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kRows;
+  const int Rw = R0 + 16 * rg + c;
+  if (R0 >= nrows) {  // x' only: the GEMM's padding rows qrows .. Mp - 1 as zero chunks
+    const int nch = H * (HD / 8), q0 = R0 / H, nq = kRows / H;
+    for (int i = t; i < nq * nch; i += NTH) {
+      const int qr = q0 + i % nq, ch = i / nq;
+      if (qr >= a.Mp) continue;
+      a.xt[(size_t)ch * a.Mp + qr] = make_uint4(0u, 0u, 0u, 0u);
+      a.xt[(size_t)(nch + ch) * a.Mp + qr] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    return;
+  }
+  const int Rl = (R0 + kRows < nrows ? R0 + kRows : nrows) - 1;  // the block's last live row
+  const int pos_first = sp.qpos0 + R0 / H, pos_last = sp.qpos0 + Rl / H;
+  const int kt0 = sp.kmin(a, pos_first) / kTile, kt1 = sp.kmax(pos_last) / kTile;
+  const int t0 = kt0 + (int)blockIdx.y * a.tps;
+  const int t1 = t0 + a.tps - 1 < kt1 ? t0 + a.tps - 1 : kt1;
+  if (t0 > kt1) return;
+  // this lane's row, and the tiles that any row of the wave sees
+  const bool live = Rw < nrows;
+  const int R = live ? Rw : nrows - 1;
+  const int rpos = sp.qpos0 + R / H;
+  const int rlo = a.sliding ? rpos - a.window : -1;  // keys > rlo are visible
+  const int Rf = R0 + 16 * rg < nrows ? R0 + 16 * rg : nrows - 1;
+  const int Re = R0 + 16 * rg + 15 < nrows ? R0 + 16 * rg + 15 : nrows - 1;
+  const int wt0 = R0 + 16 * rg < nrows ? sp.kmin(a, sp.qpos0 + Rf / H) / kTile : kt1 + 1;
+  const int wt1 = sp.kmax(sp.qpos0 + Re / H) / kTile;
+
+  // tiles whose every key every row of the wave sees
+  const int in0 = a.sliding ? (sp.qpos0 + Re / H - a.window) / kTile + 1 : 0;
+  const int in1 = R0 + 16 * rg + 15 < nrows ? (sp.qpos0 + Rf / H + 1) / kTile - 1 : -1;
+
+  const int base = sp.base(a);
+  auto tile = [&](int kt) { return a.kv + (size_t)(kt - base) * (20 * HD); };
+  auto load = [&](const u32x4 *src, u32x4 *dst, int pieces, int n) {
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const int u = w + WV * i < pieces ? w + WV * i : pieces - 1;  // the last one twice, same bytes
+      __builtin_amdgcn_global_load_lds((const void *)(src + u * 64 + lane), (lds_ptr)(dst + u * 64),
+                                       16, 0, 0);
+    }
+  };
+  auto load_k = [&](int kt, int sub) {
+    load(tile(kt) + sub * (6 * HD), sub ? sm.b : sm.a, KP, KW);
+  };
+  auto load_v = [&](int kt, int half) {
+    load(tile(kt) + 12 * HD + half * (4 * HD), half ? sm.b : sm.c, VP, VW);
+    if (half == 0)
+      __builtin_amdgcn_global_load_lds(
+          (const void *)(a.meta + (size_t)(kt - base) * kMetaInts + lane), (lds_ptr)sm.meta, 4, 0, 0);
+  };
+  load_k(t0, 0);
+  load_k(t0, 1);
+  load_v(t0, 0);
+
+  // q of this lane's row: dims 32 j + 8 g .. + 7, as three parts
+  bf16x8 qp[NJ][3];
+  bool qslow;
+  {
+    const float4 *src = reinterpret_cast<const float4 *>(a.q + (size_t)R * HD + dh * (HD / DH) + 8 * g);
+    float x[NJ][8];
+    uint32_t mx = 0;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const float4 u0 = src[8 * j], u1 = src[8 * j + 1];
+      x[j][0] = u0.x, x[j][1] = u0.y, x[j][2] = u0.z, x[j][3] = u0.w;
+      x[j][4] = u1.x, x[j][5] = u1.y, x[j][6] = u1.z, x[j][7] = u1.w;
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t b = __float_as_uint(x[j][i]) & 0x7fffffffu;
+        mx = b > mx ? b : mx;
+      }
+    qslow = __syncthreads_or(mx >= kBf16MaxBits);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) split8(x[j], qp[j]);
+  }
+
+  float m = -1e30f, l = 0.f;  // l: this lane's keys only
+  f32x4 o[NN];
+#pragma unroll
+  for (int n = 0; n < NN; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  for (int kt = t0; kt <= t1; ++kt) {
+    const bool mine = kt >= wt0 && kt <= wt1;
+    f16x8 ph, pl;
+    float p[8], s[8], osc = 0.f;
+    bool slow = false;
+    // the scores of 16 keys over this wave's dims: the leading products in
+    // sums of 128 dims; the pieces of two steps are read ahead
+    auto scores = [&](const u32x4 *buf, float *sc) {
+      const u32x4 *kb = buf + dh * (NJ * 3 * 64) + lane;
+      constexpr int NM = NJ > 4 ? NJ / 4 : 1;
+      f32x4 d0[NM], d1 = {0.f, 0.f, 0.f, 0.f}, d2 = d1, d3 = d1;
+#pragma unroll
+      for (int i = 0; i < NM; ++i) d0[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      bf16x8 k[NJ][3];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) k[j][i] = __builtin_bit_cast(bf16x8, kb[(j * 3 + i) * 64]);
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        f32x4 &d = d0[j % NM];
+        d1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][0], qp[j][1], d1, 0, 0, 0);
+        d2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][0], qp[j][2], d2, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][0], qp[j][0], d, 0, 0, 0);
+        d1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][1], qp[j][0], d1, 0, 0, 0);
+        d2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][1], qp[j][1], d2, 0, 0, 0);
+        d3 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][2], qp[j][0], d3, 0, 0, 0);
+      }
+      constexpr int AHEAD = 1;
+      __builtin_amdgcn_sched_group_barrier(0x100, 3 * AHEAD, 0);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+        if (j + AHEAD < NJ) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+      }
+      f32x4 d = d1 + (d2 + d3);
+#pragma unroll
+      for (int i = 0; i < NM; ++i) d += d0[i];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sc[v] = d[v];
+    };
+    if (mine) scores(sm.a, s);
+    // B has landed everywhere, and A is free
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt < t1) load_k(kt + 1, 0);
+    if (mine) {
+      scores(sm.b, s + 4);
+      if (DH > 1) {
+        sm.ex[w][0][lane] = (f32x4){s[0], s[1], s[2], s[3]};
+        sm.ex[w][1][lane] = (f32x4){s[4], s[5], s[6], s[7]};
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // B is free
+    load_v(kt, 1);
+    if (mine) {
+      if (DH > 1) {  // in dim order, so the waves of a row hold the same scores
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const f32x4 d = sm.ex[rg][u][lane] + sm.ex[rg + 4 * (DH - 1)][u][lane];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) s[4 * u + v] = d[v];
+        }
+      }
+      const bool inner = kt >= in0 && kt <= in1;
+      slow = qslow || __builtin_amdgcn_readfirstlane(sm.meta[33] | sm.meta[34]) != 0;
+      auto key_of = [&](int i) { return kt * kTile + (i < 4 ? 4 * g + i : 12 + 4 * g + i); };
+      if (slow) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int key = key_of(i) < sp.keylen ? key_of(i) : sp.keylen - 1;
+          const float *qf = a.q + (size_t)R * HD, *kf = a.k + (size_t)key * HD;
+          float d = 0.f;
+          for (int x = 0; x < HD; ++x) d = fmaf(qf[x], kf[x], d);
+          s[i] = d;
+        }
+      }
+      if (!inner) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int key = key_of(i);
+          if (!(live && key <= rpos && key < sp.keylen && key > rlo)) s[i] = -INFINITY;
+        }
+      }
+      float tm = s[0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) tm = fmaxf(tm, s[i]);
+      // the running maximum in units of log 2: p = 2^(s log2 e - m), one
+      // rounding of the exponent's argument.  (fmaxf drops a NaN score, whose
+      // p is NaN.)
+      const float mn = fmaxf(m, group_max(tm) * kLog2e);
+      const float corr = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      const f32x4 f0 = *reinterpret_cast<const f32x4 *>(&sm.meta[4 * g]);
+      const f32x4 f1 = *reinterpret_cast<const f32x4 *>(&sm.meta[16 + 4 * g]);
+      const int em = sm.meta[32];
+      float ls = 0.f, pm = 0.f, x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        p[i] = __builtin_amdgcn_exp2f(fmaf(s[i], kLog2e, -mn));  // 0 for a masked key
+        ls += p[i];
+        x[i] = p[i] * (i < 4 ? f0[i & 3] : f1[i & 3]);
+        pm = fmaxf(pm, x[i]);
+      }
+      l = fmaf(l, corr, ls);
+      int z = 14 - __builtin_amdgcn_frexp_expf(group_max(pm));
+      z = z < 100 ? z : 100;
+      osc = ldexpf(1.f, em - z);
+      const float zf = ldexpf(1.f, z);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float y = x[i] * zf;
+        ph[i] = (_Float16)y;
+        pl[i] = (_Float16)(y - (float)ph[i]);
+      }
+      if (__any(corr != 1.f)) {
+#pragma unroll
+        for (int n = 0; n < NN; ++n) o[n] *= corr;
+      }
+    }
+    auto outputs = [&](const u32x4 *buf, auto half) {
+      constexpr int n0 = decltype(half)::value * (NN / 2);
+      const u32x4 *vb = buf + dh * (NN * 64) + lane;
+      f16x8 vv[NN / 2][2];
+#pragma unroll
+      for (int i = 0; i < NN / 2; ++i) {
+        vv[i][0] = __builtin_bit_cast(f16x8, vb[(2 * i) * 64]);
+        vv[i][1] = __builtin_bit_cast(f16x8, vb[(2 * i + 1) * 64]);
+      }
+#pragma unroll
+      for (int i = 0; i < NN / 2; i += 2) {
+        f32x4 d[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          d[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[i + u][1], ph, (f32x4){0.f, 0.f, 0.f, 0.f},
+                                                        0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          d[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[i + u][0], pl, d[u], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          d[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[i + u][0], ph, d[u], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) o[n0 + i + u][v] = fmaf(d[u][v], osc, o[n0 + i + u][v]);
+      }
+      constexpr int AHEAD = 2;
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * AHEAD, 0);
+#pragma unroll
+      for (int i = 0; i < NN / 2; i += 2) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+        if (i + AHEAD < NN / 2) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+        if (i > 0) __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+      }
+    };
+    if (mine && !slow) outputs(sm.c, std::integral_constant<int, 0>());
+    // B (V) and A have landed everywhere, and C is free
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt < t1) load_v(kt + 1, 0);
+    if (mine && !slow) outputs(sm.b, std::integral_constant<int, 1>());
+    if (slow) {  // keys that the row sees, from the FP32 rows
+      for (int gg = 0; gg < 4; ++gg)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float pk = __shfl(p[i], 16 * gg + c, 64);
+          const int key = kt * kTile + (i < 4 ? 4 * gg + i : 12 + 4 * gg + i);
+          if (!(live && key <= rpos && key < sp.keylen && key > rlo)) continue;
+          const float *vp = a.v + (size_t)key * HD + dh * (HD / DH) + 4 * g;
+#pragma unroll
+          for (int n = 0; n < NN; ++n) {
+            const float4 vv = *reinterpret_cast<const float4 *>(vp + 16 * n);
+            o[n][0] = fmaf(pk, vv.x, o[n][0]);
+            o[n][1] = fmaf(pk, vv.y, o[n][1]);
+            o[n][2] = fmaf(pk, vv.z, o[n][2]);
+            o[n][3] = fmaf(pk, vv.w, o[n][3]);
+          }
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // B is free
+    if (kt < t1) load_k(kt + 1, 1);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+
+  if (gridDim.y > 1) {
+    if (!live) return;
+    float *pp = a.part + ((size_t)blockIdx.y * nrows + R) * HD + dh * (HD / DH) + 4 * g;
+#pragma unroll
+    for (int n = 0; n < NN; ++n) *reinterpret_cast<f32x4 *>(pp + 16 * n) = o[n];
+    if (g == 0 && dh == 0) a.ml[(size_t)blockIdx.y * nrows + R] = make_float2(m, l);
+    return;
+  }
+#pragma unroll
+  for (int n = 0; n < NN; ++n)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[n][v] = live ? o[n][v] / l : 0.f;
+  if (!a.xt) {
+    if (!live) return;
+    float *op = a.out + (size_t)R * HD + dh * (HD / DH) + 4 * g;
+#pragma unroll
+    for (int n = 0; n < NN; ++n) *reinterpret_cast<f32x4 *>(op + 16 * n) = o[n];
+    return;
+  }
+  // x' of the GEMM: the exponent of a query row from its H heads (H divides
+  // 16, so they are lanes of this wave); rows past qrows are zero chunks
+  float mx = 0.f;
+#pragma unroll
+  for (int n = 0; n < NN; ++n)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) mx = fmaxf(mx, fabsf(o[n][v]));
+  for (int d = 1; d < H; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  if (DH > 1) {
+    if (g == 0) sm.mx[w][c] = mx;
+    __syncthreads();
+    mx = fmaxf(sm.mx[rg][c], sm.mx[rg + 4 * (DH - 1)][c]);
+  }
+  const int e = mx > 0.f && mx <= 3.4e38f ? ilogbf(mx) - 13 : 0;
+  const int qr = Rw / H, h = Rw - qr * H;
+  if (live && h == 0 && g == 0 && dh == 0) a.xe[qr] = e;
+  const size_t lo_plane = (size_t)H * (HD / 8) * a.Mp;
+#pragma unroll
+  for (int n = 0; n < NN; ++n) {
+    const float v[4] = {o[n][0], o[n][1], o[n][2], o[n][3]};
+    const u32x4 ch = xprep_chunk(v, e, g & 1);
+    const size_t at = (size_t)(h * (HD / 8) + dh * (HD / DH / 8) + 2 * n + (g >> 1)) * a.Mp + qr + ((g & 1) ? lo_plane : 0);
+    if (qr < a.Mp) reinterpret_cast<u32x4 *>(a.xt)[at] = ch;
+  }
+}
+
+// Adds the key splits of one query row: out = sum_s 2^(m_s - M) o_s /
+// sum_s 2^(m_s - M) l_s in split order, as rows of out or as the GEMM's x'.
+// A block is one query row (x': all heads, one exponent) or one (query row,
+// head); thread t takes 16-byte units t, t + 256, ... of it.
+template <int HD, bool X>
+__global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsArgs a) {
+  constexpr int U4 = HD / 4;  // units per head
+  constexpr int kHeads = 16;
+  __shared__ float wt[X ? kHeads : 1][kMaxSplits];
+  __shared__ float rl[kHeads];
+  __shared__ float red[4];
+  const Span sp(a);
+  const int t = threadIdx.x, H = a.H, nrows = sp.nrows;
+  const int qr = X ? blockIdx.x : blockIdx.x / H, h0 = X ? 0 : blockIdx.x - qr * H;
+  const int nh = X ? H : 1;
+  if (X && qr >= a.qrows) {
+    const int nch = H * (HD / 8);
+    for (int ch = t; ch < 2 * nch; ch += 256) a.xt[(size_t)ch * a.Mp + qr] = make_uint4(0u, 0u, 0u, 0u);
+    return;
+  }
+  // splits of a row: those of its 64-row block
+  auto splits = [&](int R) {
+    const int r0 = R / kRows * kRows;
+    const int re = (r0 + kRows < nrows ? r0 + kRows : nrows) - 1;
+    const int nt = sp.kmax(sp.qpos0 + re / H) / kTile - sp.kmin(a, sp.qpos0 + r0 / H) / kTile + 1;
+    return (nt + a.tps - 1) / a.tps;
+  };
+  // weights 2^(m_s - M) and the sum of each head: 16 lanes per head
+  {
+    const int hh = t >> 4, li = t & 15;
+    const int R = qr * H + h0 + (hh < nh ? hh : 0), ns = splits(R);
+    float2 ml[kMaxSplits / 16];
+    float M = -2e30f, L = 0.f;
+#pragma unroll
+    for (int i = 0; i < kMaxSplits / 16; ++i) {
+      const int s = li + 16 * i;
+      ml[i] = a.ml[(size_t)(s < ns ? s : 0) * nrows + R];
+      M = fmaxf(M, ml[i].x);
+    }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+#pragma unroll
+    for (int i = 0; i < kMaxSplits / 16; ++i) {
+      const int s = li + 16 * i;
+      const float e = s < ns ? __builtin_amdgcn_exp2f(ml[i].x - M) : 0.f;
+      if (hh < nh) wt[hh][s] = e;
+      L += s < ns ? e * ml[i].y : 0.f;
+    }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) L += __shfl_xor(L, o, 64);
+    if (hh < nh && li == 0) rl[hh] = L;
+  }
+  __syncthreads();
+  constexpr int NU = X ? kHeads * U4 / 256 : (U4 + 255) / 256;
+  f32x4 v[NU];
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < NU; ++i) {
+    v[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int u = t + 256 * i, h = u / U4, d = u - h * U4;
+    if (h >= nh) continue;
+    const int R = qr * H + h0 + h, ns = splits(R);
+    const float *p = a.part + (size_t)R * HD + 4 * d;
+    const size_t step = (size_t)nrows * HD;
+    int s = 0;
+    for (; s + 4 <= ns; s += 4) {
+      f32x4 x[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[k] = *reinterpret_cast<const f32x4 *>(p + (s + k) * step);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[i] += wt[h][s + k] * x[k];
+    }
+    for (; s < ns; ++s) v[i] += wt[h][s] * *reinterpret_cast<const f32x4 *>(p + s * step);
+    const float L = rl[h];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[i][k] = v[i][k] / L;
+      mx = fmaxf(mx, fabsf(v[i][k]));
+    }
+    if (!X) *reinterpret_cast<f32x4 *>(a.out + (size_t)R * HD + 4 * d) = v[i];
+  }
+  if (!X) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  if ((t & 63) == 0) red[t >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const int e = mx > 0.f && mx <= 3.4e38f ? ilogbf(mx) - 13 : 0;
+  if (t == 0) a.xe[qr] = e;
+  const size_t lo_plane = (size_t)H * (HD / 8) * a.Mp;
+#pragma unroll
+  for (int i = 0; i < NU; ++i) {
+    const int u = t + 256 * i;  // units 2 ch and 2 ch + 1 sit in neighbouring lanes
+    _Float16 hv[4], lv[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float s = ldexpf(v[i][k], -e);
+      hv[k] = (_Float16)s;
+      lv[k] = (_Float16)(s - (float)hv[k]);
+    }
+    const bool odd = t & 1;
+    const uint32_t h01 = pack_h2(hv[0], hv[1]), h23 = pack_h2(hv[2], hv[3]);
+    const uint32_t l01 = pack_h2(lv[0], lv[1]), l23 = pack_h2(lv[2], lv[3]);
+    const uint32_t r01 = __shfl_xor(odd ? h01 : l01, 1, 64);
+    const uint32_t r23 = __shfl_xor(odd ? h23 : l23, 1, 64);
+    const uint32_t a01 = odd ? r01 : h01, a23 = odd ? r23 : h23;
+    const uint32_t b01 = odd ? l01 : r01, b23 = odd ? l23 : r23;
+    if (u / U4 < nh)
+      reinterpret_cast<u32x4 *>(a.xt)[(size_t)(u >> 1) * a.Mp + qr + (odd ? lo_plane : 0)] =
+          (u32x4){(a01 & 0xffffu) | (b01 << 16), (a01 >> 16) | (b01 & 0xffff0000u),
+                  (a23 & 0xffffu) | (b23 << 16), (a23 >> 16) | (b23 & 0xffff0000u)};
+  }
+}
+
+int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+struct RowsPlan {
+  int tiles, tps, splits;
+  size_t kv, meta, part, total;  // floats
+};
+
+int cus() { return cu_count() > 0 ? cu_count() : 256; }
+
+// Most keys that the rows of `positions` consecutive positions see.
+int keys_seen(int positions, int max_keylen, bool sliding, int window) {
+  const long n = (long)window - 1 + positions;
+  return sliding && n < max_keylen ? (int)n : max_keylen;
+}
+
+// Key tiles of the call, and the split of a row block's tiles over blocks:
+// as many as fill the CUs (one block per CU at head dim 512, two below), at
+// least two tiles each, and no more than `avail` floats of scratch hold.
+bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int window,
+               size_t avail, RowsPlan *p) {
+  const int nrows = qrows * heads, blocks = cdiv(nrows, kRows);
+  const int span = cdiv(kRows, heads) + 1;  // positions of a block's rows
+  const int all = cdiv(max_keylen, kTile);
+  auto tiles_of = [&](int positions) {  // whatever their alignment
+    const int n = (keys_seen(positions, max_keylen, sliding, window) + kTile - 2) / kTile + 1;
+    return n < all ? n : all;
+  };
+  p->tiles = tiles_of(qrows);
+  const int nt = tiles_of(span < qrows ? span : qrows);
+  int splits = (hd > 256 ? 1 : 2) * cus() / blocks;
+  if (splits > kMaxSplits) splits = kMaxSplits;
+  p->kv = (size_t)p->tiles * hd * 80;
+  p->meta = (size_t)p->tiles * kMetaInts;
+  for (;; --splits) {
+    p->tps = splits > 1 ? cdiv(nt, splits) : nt;
+    if (p->tps < 2) p->tps = 2;
+    p->splits = cdiv(nt, p->tps);
+    p->part = p->splits > 1 ? (size_t)p->splits * nrows * (hd + 2) : 0;
+    p->total = p->kv + p->meta + p->part;
+    if (p->total <= avail) return true;
+    if (splits <= 1) return false;
+  }
+}
+
+template <int HD>
+int launch_rows(const RowsArgs &a, const RowsPlan &p) {
+  hipLaunchKernelGGL(attn_kv_split_kernel<HD>, dim3(p.tiles, 2), dim3(512), 0, stream(), a);
+  G4_LAUNCH_CHECK("attn_kv_split_kernel");
+  const bool pad = a.xt && p.splits == 1;
+  const dim3 grid(cdiv((pad ? a.Mp : a.qrows) * a.H, kRows), p.splits);
+  hipLaunchKernelGGL(attn_rows_f16_kernel<HD>, grid, dim3(256 * kDimWaves<HD>), 0, stream(), a);
+  G4_LAUNCH_CHECK("attn_rows_f16_kernel");
+  if (p.splits == 1) return G4_OK;
+  if (a.xt)
+    hipLaunchKernelGGL((attn_rows_merge_kernel<HD, true>), dim3(a.Mp), dim3(256), 0, stream(), a);
+  else
+    hipLaunchKernelGGL((attn_rows_merge_kernel<HD, false>), dim3(a.qrows * a.H), dim3(256), 0,
+                       stream(), a);
+  G4_LAUNCH_CHECK("attn_rows_merge_kernel");
+  return G4_OK;
+}
+
+}  // namespace
+
+// Where the FP32 matrix kernels take longer: their time is that of the heaviest
+// 16-row block's walk over 16-key tiles (about 1.6 us a tile at head dim 512,
+// 0.75 at 256) times the rounds of such blocks over the CUs, and 10 us.  Here a
+// call costs 25 to 35 us before keys matter (three launches, q's conversion
+// and, growing with the rows, the planes of the key splits).  Measured at 8
+// heads, FP32 kernel against this one: head dim 512, 12 rows over 212 keys
+// 31.4 / 31.2 us, 362 keys 47 / 33, 80 rows over 280 keys 39 / 36, 256 rows over
+// 256 keys 35 / 39; head dim 256, 20 rows over 220 keys 21 / 23, 370 keys 27 / 24,
+// 512 rows over 512 keys 33 / 39, 700 rows over 700 keys 51 / 45.
+bool attention_rows_wins(int qrows, int heads, int hd, int max_keylen, bool sliding, int window) {
+  if (hd != 256 && hd != 512) return false;
+  const int nrows = qrows * heads;
+  const int keys = keys_seen(cdiv(16, heads) + 1, max_keylen, sliding, window);
+  const int steps = cdiv(keys, 16) * cdiv(nrows, 16 * cus());
+  return hd == 512 ? steps >= 18 : steps >= 22 + nrows / 200;
+}
+
+size_t attention_rows_floats(int qrows, int heads, int hd, int max_keylen, bool sliding,
+                             int window) {
+  RowsPlan p;
+  if (!attention_rows_wins(qrows, heads, hd, max_keylen, sliding, window)) return 0;
+  rows_plan(qrows, heads, hd, max_keylen, sliding, window, ~size_t(0), &p);
+  return p.total;
+}
+
+int launch_attention_rows(const float *q, const float *k, const float *v, int qrows, int heads,
+                          int hd, int keylen, int qpos0, const int *pos_dev, int max_keylen,
+                          bool sliding, int window, float *scratch, size_t scratch_floats,
+                          float *out, void *xt, int *xe, int Mp, bool *taken) {
+  RowsPlan p;
+  *taken = false;
+  if (!rows_plan(qrows, heads, hd, max_keylen, sliding, window, scratch_floats, &p)) return G4_OK;
+  RowsArgs a{};
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.out = out;
+  a.xt = static_cast<uint4 *>(xt);
+  a.xe = xe;
+  a.Mp = Mp;
+  a.kv = reinterpret_cast<u32x4 *>(scratch);
+  a.meta = reinterpret_cast<int *>(scratch + p.kv);
+  a.part = scratch + p.kv + p.meta;
+  a.ml = reinterpret_cast<float2 *>(a.part + (size_t)p.splits * qrows * heads * hd);
+  a.H = heads;
+  a.hd = hd;
+  a.keylen = keylen;
+  a.qpos0 = qpos0;
+  a.sliding = sliding ? 1 : 0;
+  a.window = window;
+  a.qrows = qrows;
+  a.tps = p.tps;
+  a.pos_dev = pos_dev;
+  *taken = true;
+  return hd == 512 ? launch_rows<512>(a, p) : launch_rows<256>(a, p);
+}
+
+}  // namespace g4

@@ -235,7 +235,8 @@ int run_token(g4_gemma *m, bool graph) {
                                 l.rope_base, eps, m->q, l.kc, l.vc, own)))
         return rc;
       if ((rc = launch_attention(m->q, src.kc, src.vc, 1, c.heads, l.hd, keylen_host, 0, m->pos,
-                                 max_keylen, !l.full, c.window, kpw_for(1), m->part, m->ctx)))
+                                 max_keylen, !l.full, c.window, kpw_for(1), m->part,
+                                 m->part_floats, m->ctx)))
         return rc;
     }
     if ((rc = g4_w4_linear(l.w[G4_PROJ_O], m->ctx, G4_F32, 1, m->attn, G4_F32))) return rc;
@@ -403,8 +404,8 @@ int run_layers(g4_gemma *m, int rows, bool graph, const Diag *dg = nullptr) {
     bool o_prepped = false;
     if (gemm && (rc = w4_gemm_prepare(&ow, 1, rows, &oxp))) return rc;
     if ((rc = launch_attention(m->q, src.kc, src.vc, rows, c.heads, l.hd, keylen_host, 0, m->pos,
-                               max_keylen, !l.full, c.window, kpw, m->part, m->ctx, oxp.xt,
-                               oxp.xe, oxp.Mp, gemm ? &o_prepped : nullptr)))
+                               max_keylen, !l.full, c.window, kpw, m->part, m->part_floats,
+                               m->ctx, oxp.xt, oxp.xe, oxp.Mp, gemm ? &o_prepped : nullptr)))
       return rc;
     if (sb && (rc = stage(G4_STAGE_ATTENTION_CONTEXT, m->ctx))) return rc;
     GemmParts op;

@@ -30,7 +30,9 @@ int launch_norm_rope_qkv(const float *q, int qparts, size_t qpstride, const floa
                          const float *v, int rows, int heads, int hd, const int *pos_dev,
                          const float *qscale, const float *kscale, int rope_angles, float base,
                          float eps, float *qy, float *kc, float *vc);
-// Floats of split scratch that launch_attention needs for up to max_keylen keys.
+// Floats of split scratch that launch_attention needs for up to max_keylen keys
+// (part_floats at least; with fewer than attention_rows_floats many query rows
+// take the slower matrix-core kernel).
 size_t attention_part_floats(int qrows, int heads, int hd, int max_keylen, int kpw);
 // With xt, xe, Mp (w4_gemm_prepare of the GEMM that takes the [qrows, heads
 // * hd] output) and x_done: where the matrix-core kernel runs and its 16-row
@@ -38,8 +40,19 @@ size_t attention_part_floats(int qrows, int heads, int hd, int max_keylen, int k
 // GEMM's x' instead of through `out`, and *x_done is set.
 int launch_attention(const float *q, const float *k, const float *v, int qrows, int heads,
                      int hd, int keylen, int qpos0, const int *pos_dev, int max_keylen,
-                     bool sliding, int window, int kpw, float *part, float *out,
-                     void *xt = nullptr, int *xe = nullptr, int Mp = 0, bool *x_done = nullptr);
+                     bool sliding, int window, int kpw, float *part, size_t part_floats,
+                     float *out, void *xt = nullptr, int *xe = nullptr, int Mp = 0, bool *x_done = nullptr);
+// launch_attention's form for many query rows over long caches
+// (g4_attn_rows.hip): whether it is the faster one, the scratch floats it asks
+// for (0 where it is not), and its launch.  *taken is cleared, and nothing
+// launched, where scratch_floats do not hold its split tiles.  xt / xe / Mp as above (heads divides 16, Mp a multiple of 16).
+bool attention_rows_wins(int qrows, int heads, int hd, int max_keylen, bool sliding, int window);
+size_t attention_rows_floats(int qrows, int heads, int hd, int max_keylen, bool sliding,
+                             int window);
+int launch_attention_rows(const float *q, const float *k, const float *v, int qrows, int heads,
+                          int hd, int keylen, int qpos0, const int *pos_dev, int max_keylen,
+                          bool sliding, int window, float *scratch, size_t scratch_floats,
+                          float *out, void *xt, int *xe, int Mp, bool *taken);
 int launch_ple_mix(const float *proj, float pre_scale, const float *norm_scale,
                    const float *token_ple, int rows, int width, int layers, float eps,
                    float ple_scale, float out_scale, float *y);

@@ -1264,8 +1264,8 @@ int launch_combine(const float *part, int heads, int hd, int kpw, int nsplit, in
 
 int launch_attention(const float *q, const float *k, const float *v, int qrows, int heads,
                      int hd, int keylen, int qpos0, const int *pos_dev, int max_keylen,
-                     bool sliding, int window, int kpw, float *part, float *out, void *xt,
-                     int *xe, int Mp, bool *x_done) {
+                     bool sliding, int window, int kpw, float *part, size_t part_floats,
+                     float *out, void *xt, int *xe, int Mp, bool *x_done) {
   if (x_done) *x_done = false;
   if (qrows == 0) return G4_OK;
   if (max_keylen > kDecMaxKeys * kMaxSplits)
@@ -1285,6 +1285,18 @@ int launch_attention(const float *q, const float *k, const float *v, int qrows, 
     }
     G4_LAUNCH_CHECK("attn_dec_kernel");
     return launch_combine(part, heads, hd, 0, ns, keylen, pos_dev, qrows, out);
+  }
+  // x' for the next GEMM when asked for and 16 rows hold whole query rows
+  const bool xprep = xt && x_done && kFaRows % heads == 0 && Mp >= qrows && Mp % 16 == 0;
+  if (attention_rows_wins(qrows, heads, hd, max_keylen, sliding, window)) {
+    bool taken;
+    const int rc = launch_attention_rows(q, k, v, qrows, heads, hd, keylen, qpos0, pos_dev,
+                                         max_keylen, sliding, window, part, part_floats, out,
+                                         xprep ? xt : nullptr, xe, Mp, &taken);
+    if (rc || taken) {
+      if (!rc && xprep) *x_done = true;
+      return rc;
+    }
   }
   kpw = split_kpw(kpw, max_keylen);
   AttnArgs a;
@@ -1309,9 +1321,7 @@ int launch_attention(const float *q, const float *k, const float *v, int qrows, 
   // Many rows, or few keys: the matrix-core kernel (16 rows per block, no
   // merge pass).  A handful of rows over a long cache keeps the key split.
   if ((size_t)qrows * heads >= 64 || max_keylen <= 512) {
-    // x' for the next GEMM when asked for and the block's 16 rows hold whole
-    // query rows; the grid then also covers the GEMM's padding rows
-    const bool xprep = xt && x_done && kFaRows % heads == 0 && Mp >= qrows && Mp % 16 == 0;
+    // with x', the grid also covers the GEMM's padding rows
     if (xprep) {
       a.xt = static_cast<uint4 *>(xt);
       a.xe = xe;
@@ -1483,11 +1493,15 @@ G4_API int g4_attention(const float *q, const float *k, const float *v, int qrow
   if (rc) return rc;
   const int kpw = attn_kpw(qrows);
   void *part = nullptr;
-  rc = g_attn_ws.get(attention_part_floats(qrows, heads, head_dim, keylen, kpw) * 4, &part,
-                     "g4_attention");
+  size_t floats = attention_part_floats(qrows, heads, head_dim, keylen, kpw);
+  const size_t more = attention_rows_floats(qrows, heads, head_dim, keylen, sliding != 0, window);
+  // a recording takes the scratch that is there, if it is enough to run at all
+  if (more > floats && !(encoding() && g_attn_ws.bytes < more * 4)) floats = more;
+  rc = g_attn_ws.get(floats * 4, &part, "g4_attention");
   if (!rc)
     rc = launch_attention(q, k, v, qrows, heads, head_dim, keylen, qpos0, nullptr, keylen,
-                          sliding != 0, window, kpw, static_cast<float *>(part), y);
+                          sliding != 0, window, kpw, static_cast<float *>(part),
+                          g_attn_ws.bytes / 4, y);
   return rc ? rc : ok();
 }
 

@@ -224,6 +224,95 @@ def test_attention_rows_cache_longer_than_keylen(g4, qrows):
     check_attention(got, want, fp32_attention(q, k, v, qrows, heads, hd, keylen, qpos0, True, 16))
 
 
+def rows_case(qrows, heads, hd, keylen, tail, seed, spread=0.0):
+    """q/k/v of an attention over `keylen` keys whose last `tail` lie past the last query row;
+    spread: row magnitudes 10^(+-spread)."""
+    rng = np.random.default_rng([seed, qrows, heads, hd, keylen])
+    q = rng.standard_normal((qrows, heads * hd)).astype(np.float32) * np.float32(hd ** -0.25)
+    k = rng.standard_normal((keylen, hd)).astype(np.float32) * np.float32(hd ** -0.25)
+    v = rng.standard_normal((keylen, hd)) * 10.0 ** rng.uniform(-spread, spread, (keylen, 1))
+    return q, k, v.astype(np.float32), keylen - tail - qrows
+
+
+def run_attention(g4, q, k, v, qrows, heads, hd, keylen, qpos0, sliding, window):
+    y = out(g4, qrows * heads * hd)
+    g4.attention(dev(g4, q), dev(g4, k), dev(g4, v), qrows, heads, hd, keylen, qpos0, sliding,
+                 window, y)
+    return y.download(np.float32).reshape(qrows, heads * hd)
+
+
+# Many query rows over long caches (the split-operand kernel): tile edges of its
+# 32 keys and 64 rows, its key splits (few rows) and none (many), windows off the
+# tile grid, head counts that do and do not divide 64, keys past the last row.
+@pytest.mark.parametrize("qrows,heads,hd,keylen,tail,sliding,window", [
+    (2, 8, 512, 289, 0, False, 0), (2, 1, 512, 320, 31, False, 0), (5, 3, 512, 321, 1, False, 0),
+    (9, 8, 512, 1000, 0, True, 333), (33, 8, 512, 545, 32, False, 0), (40, 5, 512, 290, 0, True, 511),
+    (2, 8, 256, 353, 0, False, 0), (3, 7, 256, 900, 65, True, 512), (17, 8, 256, 416, 0, False, 0),
+    (64, 4, 256, 1057, 0, True, 500), (700, 8, 256, 700, 0, True, 512), (513, 8, 512, 513, 0, True, 300),
+    (1100, 8, 256, 1100, 0, False, 0),
+])
+def test_attention_rows_over_long_caches(g4, qrows, heads, hd, keylen, tail, sliding, window):
+    q, k, v, qpos0 = rows_case(qrows, heads, hd, keylen, tail, 21)
+    k[qpos0 + qrows:] = np.nan  # never read
+    v[qpos0 + qrows:] = np.nan
+    got = run_attention(g4, q, k, v, qrows, heads, hd, keylen, qpos0, sliding, window)
+    n = qpos0 + qrows
+    want = lo.attention(q, k[:n], v[:n], qrows, heads, hd, n, qpos0, sliding, window)
+    check_attention(got, want, fp32_attention(q, k[:n], v[:n], qrows, heads, hd, n, qpos0, sliding,
+                                              window))
+
+
+@pytest.mark.parametrize("hd", [256, 512])
+def test_attention_rows_value_rows_of_any_size(g4, hd):
+    # value rows from 1e-18 to 1e18 (each has its own exponent).  Per element the
+    # error is a few roundings of sum p |v|: 22-bit halves of p and v (3 x 2^-22)
+    # and the p of scores rounded at 2^-24 |s| with |s| < 8, about 2^-20 in all.
+    qrows, heads, keylen = 12, 8, 600
+    q, k, v, qpos0 = rows_case(qrows, heads, hd, keylen, 0, 22, spread=18.0)
+    got = run_attention(g4, q, k, v, qrows, heads, hd, keylen, qpos0, False, 0)
+    want = lo.attention(q, k, v, qrows, heads, hd, keylen, qpos0, False, 0)
+    size = lo.attention(q, k, np.abs(v), qrows, heads, hd, keylen, qpos0, False, 0)
+    assert np.all(np.abs(got - want) <= 2.0 ** -19 * size)
+
+
+@pytest.mark.parametrize("hd", [256, 512])
+def test_attention_rows_nonfinite_stay_with_the_rows_that_see_them(g4, hd):
+    qrows, heads, keylen = 20, 8, 620
+    q, k, v, qpos0 = rows_case(qrows, heads, hd, keylen, 0, 23)
+    bad = qpos0 + 7  # rows 0 .. 6 do not see it
+    for where in ("v", "k", "q"):
+        a = {"q": q.copy(), "k": k.copy(), "v": v.copy()}
+        if where == "q":
+            a["q"][7, :hd] = np.inf  # head 0 of row 7
+        else:
+            a[where][bad, 3] = np.nan
+        got = run_attention(g4, a["q"], a["k"], a["v"], qrows, heads, hd, keylen, qpos0, False, 0)
+        want = lo.attention(q, k, v, qrows, heads, hd, keylen, qpos0, False, 0)
+        hit = np.zeros((qrows, heads * hd), bool)
+        if where == "q":
+            hit[7, :hd] = True
+        elif where == "k":
+            hit[7:] = True
+        else:
+            hit[7:, 3::hd] = True
+        assert np.all(np.isnan(got[hit]))
+        np.testing.assert_allclose(got[~hit], want[~hit], rtol=2e-5, atol=1e-5)
+
+
+def test_attention_rows_recorded_equals_eager(g4):
+    qrows, heads, hd, keylen = 24, 8, 512, 500
+    q, k, v, qpos0 = rows_case(qrows, heads, hd, keylen, 0, 24)
+    eager = run_attention(g4, q, k, v, qrows, heads, hd, keylen, qpos0, False, 0)
+    b = [dev(g4, a) for a in (q, k, v)]
+    y = out(g4, eager.size)
+    with g4.Encoder() as enc:
+        g4.attention(b[0], b[1], b[2], qrows, heads, hd, keylen, qpos0, False, 0, y)
+    for _ in range(3):
+        enc.cmdbuf.submit()
+        np.testing.assert_array_equal(y.download(np.float32).reshape(eager.shape), eager)
+        run_attention(g4, k[:4, :hd].repeat(heads, 1), v, k, 4, heads, hd, keylen, 400, False, 0)
+
+
 # One row's key splits: 64 and fewer, more, and more than one round of loads holds.
 @pytest.mark.parametrize("hd,keylen", [(256, 1024), (256, 1040), (512, 4097), (64, 6000)])
 def test_attention_one_row_many_splits(g4, hd, keylen):
