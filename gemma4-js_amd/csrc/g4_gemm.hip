@@ -994,6 +994,21 @@ size_t splitk_pstride(const g4_w4 *const *w, int nw, int rows) {
   return (n + 63) & ~size_t(63);
 }
 
+int launch_splitk_sum(const float *part, int slices, size_t pstride, size_t n, void *y,
+                      bool y_bf16) {
+  const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+  const size_t threads = vec ? n / 4 : n;
+  const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
+  if (vec)
+    hipLaunchKernelGGL(gemm_splitk_sum_kernel<true>, grid, dim3(kThreads), 0, stream(), part, slices,
+                       pstride, n, y, (int)y_bf16);
+  else
+    hipLaunchKernelGGL(gemm_splitk_sum_kernel<false>, grid, dim3(kThreads), 0, stream(), part,
+                       slices, pstride, n, y, (int)y_bf16);
+  G4_LAUNCH_CHECK("gemm_splitk_sum_kernel");
+  return G4_OK;
+}
+
 // n weights (1..kMaxGemmSegs) of one input dimension, y[i] receiving weight
 // i's output; a K split (slices > 1) that is summed here takes one weight,
 // one left to the caller (sum false) any number.
@@ -1031,21 +1046,8 @@ int launch_gemm(const g4_w4 *const *w, int nw, const uint4 *xt, const int *xe, i
                      reinterpret_cast<const u32x4 *>(xt), xe, sg, (int)y_bf16, rows, Mp,
                      w[0]->K, xcd_map, part, pstride);
   G4_LAUNCH_CHECK("w4_gemm_kernel");
-  if (slices > 1 && sum) {
-    void *y = ys[0];
-    const size_t n = (size_t)rows * w[0]->N;
-    const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-    const size_t threads = vec ? n / 4 : n;
-    const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
-    if (vec)
-      hipLaunchKernelGGL(gemm_splitk_sum_kernel<true>, grid, dim3(kThreads), 0, stream(), part,
-                         slices, pstride, n, y, (int)y_bf16);
-    else
-      hipLaunchKernelGGL(gemm_splitk_sum_kernel<false>, grid, dim3(kThreads), 0, stream(), part,
-                         slices, pstride, n, y, (int)y_bf16);
-    G4_LAUNCH_CHECK("gemm_splitk_sum_kernel");
-  }
-  return G4_OK;
+  return slices > 1 && sum ? launch_splitk_sum(part, slices, pstride, (size_t)rows * w[0]->N, ys[0], y_bf16)
+                           : G4_OK;
 }
 
 // The registers-B kernel: BM = 16 TMW rows by BN = 64 TNW columns per block,
@@ -1089,21 +1091,8 @@ int launch_gemm_rb(const g4_w4 *const *w, int nw, const uint4 *xt, const int *xe
                      0, stream(), reinterpret_cast<const u32x4 *>(xt), xe, sg, (int)y_bf16, rows,
                      Mp, w[0]->K, xcd_map, part, pstride);
   G4_LAUNCH_CHECK("w4_gemm_rb_kernel");
-  if (slices > 1 && sum) {
-    void *y = ys[0];
-    const size_t n = (size_t)rows * w[0]->N;
-    const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-    const size_t threads = vec ? n / 4 : n;
-    const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
-    if (vec)
-      hipLaunchKernelGGL(gemm_splitk_sum_kernel<true>, grid, dim3(kThreads), 0, stream(), part,
-                         slices, pstride, n, y, (int)y_bf16);
-    else
-      hipLaunchKernelGGL(gemm_splitk_sum_kernel<false>, grid, dim3(kThreads), 0, stream(), part,
-                         slices, pstride, n, y, (int)y_bf16);
-    G4_LAUNCH_CHECK("gemm_splitk_sum_kernel");
-  }
-  return G4_OK;
+  return slices > 1 && sum ? launch_splitk_sum(part, slices, pstride, (size_t)rows * w[0]->N, ys[0], y_bf16)
+                           : G4_OK;
 }
 
 // Tile and K split of one prefill GEMM.  Tile: the largest (128 x 128, BF16
@@ -1214,6 +1203,8 @@ namespace g4 {
 // The GEMM scratch for one call: x' planes, row exponents and K-slice planes.
 struct GemmScratch {
   GemmPlan plan;
+  bool few;  // the few-row kernel takes the call, by `small`
+  GemmSmallPlan small;
   int Mp;
   uint4 *xt;
   int *xe;
@@ -1232,32 +1223,52 @@ void xprep_layout(int K, int rows, bool f32x, int *Mp, size_t *eoff, size_t *xen
   *xend = *eoff + (size_t)rows * 4;
 }
 
+size_t part_bytes(const g4_w4 *const *w, int nw, int rows, int slices) {
+  return slices > 1 ? slices * splitk_pstride(w, nw, rows) * 4 : 0;
+}
+
 int gemm_scratch(const g4_w4 *const *w, int nw, bool f32x, int rows, bool prepped,
-                 GemmScratch *sc, const ExtScratch *ext, bool multi_split = false) {
+                 GemmScratch *sc, const ExtScratch *ext, bool multi_split, bool sum, bool glu) {
   const g4_w4 *w0 = w[0];
   size_t eoff, xend;
   xprep_layout(w0->K, rows, f32x, &sc->Mp, &eoff, &xend);
   const size_t poff = prepped ? 0 : (xend + 255) & ~size_t(255);
   sc->plan = plan_gemm(w, nw, rows, f32x, multi_split);
-  const size_t part_bytes =
-      sc->plan.slices > 1 ? sc->plan.slices * splitk_pstride(w, nw, rows) * 4 : 0;
+  size_t need = poff + part_bytes(w, nw, rows, sc->plan.slices);
+  // with x' prepared there is no pre-pass to save, only the wait per stage: the
+  // engine's prompts (us saved per prompt of 37 / 128 / 301 / 512 tokens: 790 /
+  // 760 / 170 / -170) take it up to 384 rows
+  sc->few = (!prepped || rows <= 384) && gemm_small_plan(w, nw, rows, glu, sum, &sc->small);
+  // the few-row kernel converts x itself: its planes take the place of x'
+  const size_t few = sc->few ? part_bytes(w, nw, rows, sc->small.slices) : 0;
+  if (prepped && few > need) need = few;
+  if (few > need) sc->few = false;
   void *ws = nullptr, *wx = nullptr;
   if (ext) {
     // one region: x', exponents, then the K-slice planes (x is never prepared here)
     if (prepped) return fail(G4_E_ARG, "%s: a prepared x needs the library scratch", ext->who);
-    if (poff + part_bytes > ext->bytes)
+    if (need > ext->bytes)
       return fail(G4_E_ARG,
                   "%s: %d rows of in_dim %d (%s x) into out_dim %d need %zu bytes of scratch; "
                   "the static scratch holds %zu",
-                  ext->who, rows, w0->K, f32x ? "FP32" : "BF16", w0->N, poff + part_bytes,
-                  ext->bytes);
+                  ext->who, rows, w0->K, f32x ? "FP32" : "BF16", w0->N, need, ext->bytes);
     sc->xt = static_cast<uint4 *>(ext->mem);
     sc->xe = reinterpret_cast<int *>(static_cast<char *>(ext->mem) + eoff);
-    sc->part = reinterpret_cast<float *>(static_cast<char *>(ext->mem) + poff);
+    sc->part = reinterpret_cast<float *>(static_cast<char *>(ext->mem) + (sc->few ? 0 : poff));
     return G4_OK;
   }
-  if (poff + part_bytes > 0)
-    if (int rc = g_ws.get(poff + part_bytes, &ws, "g4_w4_linear (prefill)")) return rc;
+  if (sc->few && !prepped) {
+    // the scratch grows as it would for the prefill GEMM, so that what may be
+    // recorded after this call does not depend on the kernel it took; a
+    // recording needs the planes alone
+    for (int i = 0; i < nw && nw > 1; ++i) {
+      const size_t one = poff + part_bytes(w + i, 1, rows, plan_gemm(w + i, 1, rows, f32x).slices);
+      if (one > need) need = one;
+    }
+    if (encoding()) need = few;
+  }
+  if (need > 0)
+    if (int rc = g_ws.get(need, &ws, "g4_w4_linear (prefill)")) return rc;
   if (prepped) {
     if (int rc = g_ws_x.get(xend, &wx, "g4_w4_linear (prefill, prepared x)")) return rc;
   } else {
@@ -1265,7 +1276,7 @@ int gemm_scratch(const g4_w4 *const *w, int nw, bool f32x, int rows, bool preppe
   }
   sc->xt = static_cast<uint4 *>(wx);
   sc->xe = reinterpret_cast<int *>(static_cast<char *>(wx) + eoff);
-  sc->part = reinterpret_cast<float *>(static_cast<char *>(ws) + poff);
+  sc->part = reinterpret_cast<float *>(static_cast<char *>(ws) + (sc->few ? 0 : poff));
   return G4_OK;
 }
 
@@ -1279,28 +1290,40 @@ static int gemm_run(const g4_w4 *const *w, int nw, const void *x, bool f32x, int
   const int cus = cu_count() > 0 ? cu_count() : 256;
   long tiles64 = 0;
   for (int i = 0; i < nw; ++i) tiles64 += (long)((rows + 63) / 64) * ((w[i]->N + 63) / 64);
-  if (nw > 1 && tiles64 < cus && !glu && x && !keep) {
+  GemmSmallPlan few;
+  if (nw > 1 && tiles64 < cus && !glu && x && !keep &&
+      !gemm_small_plan(w, nw, rows, false, true, &few)) {
     for (int i = 0; i < nw; ++i)
       if (int rc = gemm_run(w + i, 1, x, f32x, rows, y + i, y_bf16, nullptr)) return rc;
     return G4_OK;
   }
   const g4_w4 *w0 = w[0];
   GemmScratch sc;
-  if (int rc = gemm_scratch(w, nw, f32x, rows, !x, &sc, ext, keep && nw > 1)) return rc;
+  if (int rc = gemm_scratch(w, nw, f32x, rows, !x, &sc, ext, keep && nw > 1, !keep, glu)) return rc;
   const GemmPlan plan = sc.plan;
   const int Mp = sc.Mp;
   uint4 *xt = sc.xt;
   int *xe = sc.xe;
   float *part = sc.part;
-  const bool sum = !keep || plan.slices == 1;
+  const int slices = sc.few ? sc.small.slices : plan.slices;
+  const bool sum = !keep || slices == 1;
   if (keep) {  // one entry per weight, planes side by side
     size_t off = 0;
     for (int i = 0; i < nw; ++i) {
       keep[i].parts = sum ? static_cast<const float *>(y[i]) : part + off;
-      keep[i].n = sum ? 1 : plan.slices;
+      keep[i].n = sum ? 1 : slices;
       keep[i].stride = splitk_pstride(w, nw, rows);
       off += (size_t)rows * w[i]->N;
     }
+  }
+  if (sc.few) {
+    const size_t pstride = splitk_pstride(w, nw, rows);
+    if (int rc = launch_gemm_small(sc.small, w, nw, x, f32x, xt, xe, Mp, rows, y, y_bf16, part, pstride,
+                                   glu))
+      return rc;
+    return slices > 1 && sum
+               ? launch_splitk_sum(part, slices, pstride, (size_t)rows * w0->N, y[0], y_bf16)
+               : G4_OK;
   }
   if (!x)
     return f32x ? launch_planned<2>(plan, w, nw, xt, xe, rows, Mp, y, y_bf16, part, sum, glu)
@@ -1365,6 +1388,46 @@ int w4_gemm(const g4_w4 *w, const void *x, bool f32x, int rows, void *y, bool y_
 int w4_gemm_ext(const g4_w4 *w, const void *x, bool f32x, int rows, void *y, bool y_bf16,
                 const ExtScratch &ext) {
   return gemm_run(&w, 1, x, f32x, rows, &y, y_bf16, nullptr, false, &ext);
+}
+
+// Two FP32 rows of one slice, three and four always: against the GEMV of as
+// many rows, us at K x N 1536 x 6144 and 6144 x 1536 (three slices and a sum
+// launch): two rows 6.8 / 6.7 and 8.2 / 8.8, three 8.6 / 6.8 and 13.3 / 9.2,
+// four 10.0 / 7.0 and 15.7 / 9.5; K 12288: 18.5 / 11.0, 27 / 11.5, 35.8 / 11.7.
+// With BF16 x the GEMV needs half the arithmetic and keeps up to four rows.
+static bool few_rows_plan(const g4_w4 *const *w, int nw, int rows, GemmSmallPlan *p) {
+  return gemm_small_plan(w, nw, rows, false, true, p) &&
+         (rows > 2 || p->slices == 1 || w[0]->K > 8192);
+}
+
+int w4_gemm_few(const g4_w4 *w, const void *x, int rows, void *y, bool y_bf16,
+                const ExtScratch *ext, bool *taken) {
+  GemmSmallPlan p;
+  *taken = false;
+  if (!few_rows_plan(&w, 1, rows, &p)) return G4_OK;
+  const size_t need = part_bytes(&w, 1, rows, p.slices);
+  void *ws = nullptr;
+  // the GEMV needs no scratch: it stays where none can be had
+  if (ext) {
+    if (need > ext->bytes) return G4_OK;
+    ws = ext->mem;
+  } else if (need > 0) {
+    if (encoding() && g_ws.bytes < need) return G4_OK;
+    if (int rc = g_ws.get(need, &ws, "g4_w4_linear (few rows)")) return rc;
+  }
+  *taken = true;
+  float *part = static_cast<float *>(ws);
+  const size_t pstride = splitk_pstride(rows, w->N);
+  if (int rc = launch_gemm_small(p, &w, 1, x, true, nullptr, nullptr, 0, rows, &y, y_bf16, part,
+                                 pstride, false))
+    return rc;
+  return p.slices > 1 ? launch_splitk_sum(part, p.slices, pstride, (size_t)rows * w->N, y, y_bf16)
+                      : G4_OK;
+}
+
+bool w4_gemm_few_joint(const g4_w4 *const *w, int nw, int rows) {
+  GemmSmallPlan p;
+  return nw > 1 && rows > 1 && rows <= kMaxGemvRows && few_rows_plan(w, nw, rows, &p);
 }
 
 int w4_gemm_glu(const g4_w4 *gate, const g4_w4 *up, const float *x, int rows, float *act) {

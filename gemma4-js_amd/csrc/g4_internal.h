@@ -161,6 +161,12 @@ struct ExtScratch {
 };
 int w4_gemm_ext(const g4_w4 *w, const void *x, bool f32x, int rows, void *y, bool y_bf16,
                 const ExtScratch &ext);
+// 2 to kMaxGemvRows FP32 rows where the few-row matrix-core kernel beats the
+// GEMV (*taken; else nothing is launched), and whether it takes several weights
+// of one in_dim in one launch (through w4_gemm_multi).
+int w4_gemm_few(const g4_w4 *w, const void *x, int rows, void *y, bool y_bf16,
+                const ExtScratch *ext, bool *taken);
+bool w4_gemm_few_joint(const g4_w4 *const *w, int nw, int rows);
 // g4_w4_linear's argument checks and dispatch; with ext set, the GEMM path
 // uses that scratch (the GEMV paths use none).
 int w4_linear_impl(const g4_w4 *w, const void *x, int x_dtype, int rows, void *y, int y_dtype,
@@ -205,6 +211,20 @@ struct GemmXPrep {
   int Mp;
 };
 int w4_gemm_prepare(const g4_w4 *const *w, int nw, int rows, GemmXPrep *out);
+// The product for a few rows (g4_gemm_small.hip): tiles of 16 tm rows by 16 tn
+// columns, `slices` of `per` stages of K, s stages per wave.
+struct GemmSmallPlan {
+  int tm, tn, s, per, slices, groups;
+};
+// Whether the few-row kernel takes the call, and how; sum: a K split is added
+// here (one weight), not left to the caller.
+bool gemm_small_plan(const g4_w4 *const *w, int nw, int rows, bool glu, bool sum,
+                     GemmSmallPlan *p);
+// x as rows, or null: x' in xt / xe / Mp.  With slices > 1 the outputs are FP32
+// planes in part, pstride floats apart, the weights side by side.
+int launch_gemm_small(const GemmSmallPlan &p, const g4_w4 *const *w, int nw, const void *x,
+                      bool f32x, const uint4 *xt, const int *xe, int Mp, int rows, void *const *y,
+                      bool y_bf16, float *part, size_t pstride, bool glu);
 // Split-K decode GEMV of one FP32 row into per-slice partial sums
 // parts[K / 1536][N] (g4_w4.hip); returns the slice count, 0 if K does not
 // split (nothing launched), or minus a status.

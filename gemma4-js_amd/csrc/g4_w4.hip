@@ -1202,6 +1202,11 @@ int w4_linear_impl(const g4_w4 *w, const void *x, int x_dtype, int rows, void *y
   if (rows == 1 && gemv_fits && has_gemv1_plan(w->G, f32x))
     return f32x ? launch_gemv1<true>(w, x, y, y_dtype == G4_BF16)
                 : launch_gemv1<false>(w, x, y, y_dtype == G4_BF16);
+  if (f32x && rows > 1 && rows <= kMaxGemvRows && gemv_fits) {
+    bool taken;
+    const int rc2 = w4_gemm_few(w, x, rows, y, y_dtype == G4_BF16, ext, &taken);
+    if (rc2 || taken) return rc2;
+  }
   if (rows > kMaxGemvRows || !gemv_fits)
     return ext ? w4_gemm_ext(w, x, f32x, rows, y, y_dtype == G4_BF16, *ext)
                : w4_gemm(w, x, f32x, rows, y, y_dtype == G4_BF16);
@@ -1238,7 +1243,8 @@ G4_API int g4_w4_linear_multi(const g4_w4 *const *w, int n, const void *x, int x
       return fail(G4_E_ARG, "g4_w4_linear_multi: weight %d has in_dim %d, weight 0 has %d", i,
                   w[i]->K, w[0]->K);
   }
-  if (n == 1 || (rows > 1 && rows <= kMaxGemvRows) ||
+  const bool few = x_dtype == G4_F32 && w4_gemm_few_joint(w, n, rows);
+  if (n == 1 || (rows > 1 && rows <= kMaxGemvRows && !few) ||
       (rows == 1 && !has_gemv1_plan(w[0]->G, x_dtype == G4_F32))) {
     for (int i = 0; i < n; ++i)
       if (int rc = g4_w4_linear(w[i], x, x_dtype, rows, y[i], y_dtype)) return rc;

@@ -62,6 +62,73 @@ def test_random_linear(g4, seed):
                           syn.bf16_rne(got).reshape(rows, n)), (rows, n, k, f32x)
 
 
+# The few-row kernel at its edges: one to 257 stages of 64 inputs (idle waves, a
+# last slice that is short, 8 slices, one stage too many for it), row tiles of
+# 16 and 32 and several of them, ragged and tiny widths, and what it leaves to
+# the prefill GEMM and the GEMV beside it.  A wrong stage, row or column changes
+# whole elements.
+@pytest.mark.parametrize("k", [64, 128, 1536, 1600, 2048, 2112, 6144, 16384, 16448])
+@pytest.mark.parametrize("rows,n", [(2, 1), (3, 257), (4, 100), (5, 16), (16, 47), (17, 100),
+                                    (32, 33), (33, 15), (70, 240), (130, 17)])
+@pytest.mark.parametrize("f32x", [False, True])
+def test_few_rows_edges(g4, k, rows, n, f32x):
+    rng = np.random.default_rng([k, rows, n])
+    packed, scales, q = syn.w4_weights(k + 7 * rows + n, n, k)
+    lin = g4.W4Linear(packed, scales)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x *= (10.0 ** rng.uniform(-6, 6, (rows, 1))).astype(np.float32)
+    x[rows // 2] = 0.0
+    if f32x:
+        xb = g4.Buffer.from_array(x)
+    else:
+        bits = syn.bf16_rne(x)
+        xb, x = g4.Buffer.from_array(bits), syn.bf16_to_f32(bits).reshape(rows, k)
+    xd = g4.F32 if f32x else g4.BF16
+    ref = x.astype(np.float64) @ dense(q, scales).T
+    y32, y16 = g4.Buffer(rows * n * 4), g4.Buffer(rows * n * 2)
+    lin.linear(xb.ptr, xd, rows, y32.ptr, g4.F32)
+    lin.linear(xb.ptr, xd, rows, y16.ptr, g4.BF16)
+    got = y32.download(np.float32).reshape(rows, n)
+    # FP32 x to 2^-22, and one rounding (2^-24 of a partial sum, within four
+    # standard deviations 4 size) per matrix step (two per 32 inputs with FP32 x)
+    # and per slice added; up to four rows may run the GEMV, with x in two BF16
+    # parts (2^-17 per product) and as many roundings as inputs per lane
+    bound = 2.0 ** -22 + (2 * k / 32 + 16) * 2.0 ** -24
+    if rows <= 4:
+        bound += 2.0 ** -15
+    size = np.sqrt(((np.abs(x).astype(np.float64) ** 2) @ (dense(q, scales).T ** 2)))
+    assert np.all(np.abs(got - ref) <= bound * size * 4 + 1e-30), (k, rows, n, f32x)
+    assert not np.any(got[rows // 2])
+    assert np.array_equal(y16.download(np.uint16).reshape(rows, n),
+                          syn.bf16_rne(got).reshape(rows, n))
+
+
+@pytest.mark.parametrize("rows,k,widths", [(3, 1536, (70, 16)), (23, 1536, (100, 257, 16)),
+                                           (40, 2048, (64, 33)), (9, 6144, (48, 48))])
+def test_few_rows_several_weights_and_recorded(g4, rows, k, widths):
+    # several weights in one launch (one slice of K) or one by one (three slices
+    # and a sum), bit-identical to single calls and to every replay of a recording
+    lins = [g4.W4Linear(*syn.w4_weights(k + w, w, k)[:2]) for w in widths]
+    rng = np.random.default_rng(rows)
+    xb = g4.Buffer.from_array(rng.standard_normal((rows, k)).astype(np.float32))
+    one, many = ([g4.Buffer(rows * w * 4) for w in widths] for _ in range(2))
+    for lin, y in zip(lins, one):
+        lin.linear(xb.ptr, g4.F32, rows, y.ptr, g4.F32)
+    want = [y.download(np.float32) for y in one]
+    g4.W4Linear.linear_multi(lins, xb.ptr, g4.F32, rows, [y.ptr for y in many], g4.F32)
+    for y, w in zip(many, want):
+        np.testing.assert_array_equal(y.download(np.float32), w)
+    with g4.Encoder() as enc:
+        g4.W4Linear.linear_multi(lins, xb.ptr, g4.F32, rows, [y.ptr for y in many], g4.F32)
+        lins[0].linear(xb.ptr, g4.F32, rows, one[0].ptr, g4.F32)
+    for _ in range(3):
+        for y in many + one[:1]:
+            y.upload(np.zeros(y.nbytes // 4, np.float32))
+        enc.cmdbuf.submit()
+        for y, w in zip(many + one[:1], want + want[:1]):
+            np.testing.assert_array_equal(y.download(np.float32), w)
+
+
 @pytest.mark.parametrize("k", [16384, 32768])
 @pytest.mark.parametrize("rows", [1, 3, 40])
 @pytest.mark.parametrize("f32x", [False, True])
