@@ -53,6 +53,32 @@ def test_rms(g4, rows, width, with_scale):
                                atol=1e-6)
 
 
+@pytest.mark.parametrize("width", [1, 257, 2047, 2048, 2049, 5000])
+def test_rms_register_rows_and_longer_ones(g4, width):
+    # up to 2048 values of a row stay in registers, the rest is read twice
+    rng = np.random.default_rng(width)
+    x = rng.standard_normal((3, width)).astype(np.float32)
+    w = rng.standard_normal(width).astype(np.float32)
+    y = out(g4, x.size)
+    g4.rms(dev(g4, x), 3, width, dev(g4, w), y)
+    np.testing.assert_allclose(y.download(np.float32).reshape(x.shape), lo.rms(x, width, w, 1e-6),
+                               rtol=1e-5)
+
+
+@pytest.mark.parametrize("width,skip", [(8, 0), (12, 0), (2056, 0), (1536, 2), (1536, 8)])
+def test_embed_widths_and_alignment(g4, width, skip):
+    # rows of 8 values at a time, or one where the width or a table that starts
+    # `skip` values into its buffer (4 or 16 bytes) rules that out
+    rng = np.random.default_rng(width + skip)
+    bits = syn.bf16_rne(rng.standard_normal(skip + 5 * width).astype(np.float32))
+    E = dev(g4, bits)
+    ids = np.array([4, 0, 3], np.int32)
+    y = out(g4, 3 * width)
+    g4.embed(E.ptr + 2 * skip, 5, width, dev(g4, ids), 3, 2.5, y)
+    want = syn.bf16_to_f32(bits[skip:]).reshape(5, width)[ids] * np.float32(2.5)
+    np.testing.assert_array_equal(y.download(np.float32).reshape(3, width), want)
+
+
 def test_elementwise_ops(g4):
     rng = np.random.default_rng(9)
     n = 100003  # ragged: not a multiple of the block
