@@ -957,31 +957,40 @@ __global__ __launch_bounds__(kThreads, MINB) void w4_gemm_rb_kernel(
 }
 
 // y[i] = sum of part[s * pstride + i] over the slices s in order, as FP32 or
-// BF16.  VEC: four outputs per thread (n a multiple of 4, y 16-byte aligned).
+// BF16, for the weights side by side in each plane: elements off[k] .. off[k +
+// 1] - 1 go to y[k].  VEC: four outputs per thread (every off a multiple of 4,
+// every y 16-byte aligned).
+struct SumSegs {
+  void *y[kMaxGemmSegs];
+  size_t off[kMaxGemmSegs + 1];
+  int n;
+};
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void gemm_splitk_sum_kernel(const float *__restrict__ part,
                                                                    int slices, size_t pstride,
-                                                                   size_t n, void *__restrict__ y,
-                                                                   int y_bf16) {
+                                                                   SumSegs sg, int y_bf16) {
   const size_t i = ((size_t)blockIdx.x * kThreads + threadIdx.x) * (VEC ? 4 : 1);
-  if (i >= n) return;
+  if (i >= sg.off[sg.n]) return;
+  const int k = sg.n > 2 && i >= sg.off[2] ? 2 : sg.n > 1 && i >= sg.off[1] ? 1 : 0;
+  void *y = k == 2 ? sg.y[2] : k == 1 ? sg.y[1] : sg.y[0];
+  const size_t o = i - (k == 2 ? sg.off[2] : k == 1 ? sg.off[1] : 0);
   if (VEC) {
     f32x4 v = *reinterpret_cast<const f32x4 *>(part + i);
     for (int s = 1; s < slices; ++s) v += *reinterpret_cast<const f32x4 *>(part + s * pstride + i);
     if (y_bf16) {
       const uint32_t lo = f32_to_bf16_rne(v[0]) | (f32_to_bf16_rne(v[1]) << 16);
       const uint32_t hi = f32_to_bf16_rne(v[2]) | (f32_to_bf16_rne(v[3]) << 16);
-      *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + i) = make_uint2(lo, hi);
+      *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + o) = make_uint2(lo, hi);
     } else {
-      *reinterpret_cast<f32x4 *>(static_cast<float *>(y) + i) = v;
+      *reinterpret_cast<f32x4 *>(static_cast<float *>(y) + o) = v;
     }
   } else {
     float v = part[i];
     for (int s = 1; s < slices; ++s) v += part[s * pstride + i];
     if (y_bf16)
-      static_cast<uint16_t *>(y)[i] = (uint16_t)f32_to_bf16_rne(v);
+      static_cast<uint16_t *>(y)[o] = (uint16_t)f32_to_bf16_rne(v);
     else
-      static_cast<float *>(y)[i] = v;
+      static_cast<float *>(y)[o] = v;
   }
 }
 
@@ -994,29 +1003,33 @@ size_t splitk_pstride(const g4_w4 *const *w, int nw, int rows) {
   return (n + 63) & ~size_t(63);
 }
 
-int launch_splitk_sum(const float *part, int slices, size_t pstride, size_t n, void *y,
-                      bool y_bf16) {
-  const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
-  const size_t threads = vec ? n / 4 : n;
+int launch_splitk_sum(const float *part, int slices, const g4_w4 *const *w, int nw, int rows,
+                      void *const *y, bool y_bf16) {
+  SumSegs sg{};
+  sg.n = nw;
+  bool vec = true;
+  for (int i = 0; i < nw; ++i) {
+    sg.y[i] = y[i];
+    sg.off[i + 1] = sg.off[i] + (size_t)rows * w[i]->N;
+    vec = vec && sg.off[i + 1] % 4 == 0 && (reinterpret_cast<uintptr_t>(y[i]) & 15u) == 0;
+  }
+  const size_t n = sg.off[nw], threads = vec ? n / 4 : n;
   const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads));
-  if (vec)
-    hipLaunchKernelGGL(gemm_splitk_sum_kernel<true>, grid, dim3(kThreads), 0, stream(), part, slices,
-                       pstride, n, y, (int)y_bf16);
-  else
-    hipLaunchKernelGGL(gemm_splitk_sum_kernel<false>, grid, dim3(kThreads), 0, stream(), part,
-                       slices, pstride, n, y, (int)y_bf16);
+  hipLaunchKernelGGL(vec ? gemm_splitk_sum_kernel<true> : gemm_splitk_sum_kernel<false>, grid,
+                     dim3(kThreads), 0, stream(), part, slices, splitk_pstride(w, nw, rows), sg,
+                     (int)y_bf16);
   G4_LAUNCH_CHECK("gemm_splitk_sum_kernel");
   return G4_OK;
 }
 
 // n weights (1..kMaxGemmSegs) of one input dimension, y[i] receiving weight
-// i's output; a K split (slices > 1) that is summed here takes one weight,
-// one left to the caller (sum false) any number.
+// i's output; a K split (slices > 1) is summed here, or left to the caller (sum
+// false).
 template <int TM, int TN, int NX, int KS, int P>
 int launch_gemm(const g4_w4 *const *w, int nw, const uint4 *xt, const int *xe, int rows, int Mp,
                 void *const *ys, bool y_bf16, float *part, int slices, bool sum, bool glu) {
   constexpr int BM = 32 * TM, BN = 32 * TN;
-  if (Mp % BM != 0 || w[0]->G % (KS * slices) != 0 || (slices > 1 && nw != 1 && sum))
+  if (Mp % BM != 0 || w[0]->G % (KS * slices) != 0)
     return fail(G4_E_ARG, "w4_gemm: tile %dx%d (KS %d, %d slices) does not fit rows %d, K %d",
                 BM, BN, KS, slices, rows, w[0]->K);
   GemmSegs sg{};
@@ -1046,8 +1059,7 @@ int launch_gemm(const g4_w4 *const *w, int nw, const uint4 *xt, const int *xe, i
                      reinterpret_cast<const u32x4 *>(xt), xe, sg, (int)y_bf16, rows, Mp,
                      w[0]->K, xcd_map, part, pstride);
   G4_LAUNCH_CHECK("w4_gemm_kernel");
-  return slices > 1 && sum ? launch_splitk_sum(part, slices, pstride, (size_t)rows * w[0]->N, ys[0], y_bf16)
-                           : G4_OK;
+  return slices > 1 && sum ? launch_splitk_sum(part, slices, w, nw, rows, ys, y_bf16) : G4_OK;
 }
 
 // The registers-B kernel: BM = 16 TMW rows by BN = 64 TNW columns per block,
@@ -1058,8 +1070,7 @@ int launch_gemm_rb(const g4_w4 *const *w, int nw, const uint4 *xt, const int *xe
                    bool glu) {
   constexpr int BM = 16 * TMW;
   const int BN = glu ? 32 * TNW : 64 * TNW;  // output columns per block
-  if (Mp % BM != 0 || w[0]->G % (2 * slices) != 0 || (slices > 1 && nw != 1 && sum) ||
-      (glu && TNW % 2 != 0))
+  if (Mp % BM != 0 || w[0]->G % (2 * slices) != 0 || (glu && TNW % 2 != 0))
     return fail(G4_E_ARG, "w4_gemm: tile %dx%d (%d slices) does not fit rows %d, K %d", BM, BN,
                 slices, rows, w[0]->K);
   GemmSegs sg{};
@@ -1091,8 +1102,7 @@ int launch_gemm_rb(const g4_w4 *const *w, int nw, const uint4 *xt, const int *xe
                      0, stream(), reinterpret_cast<const u32x4 *>(xt), xe, sg, (int)y_bf16, rows,
                      Mp, w[0]->K, xcd_map, part, pstride);
   G4_LAUNCH_CHECK("w4_gemm_rb_kernel");
-  return slices > 1 && sum ? launch_splitk_sum(part, slices, pstride, (size_t)rows * w[0]->N, ys[0], y_bf16)
-                           : G4_OK;
+  return slices > 1 && sum ? launch_splitk_sum(part, slices, w, nw, rows, ys, y_bf16) : G4_OK;
 }
 
 // Tile and K split of one prefill GEMM.  Tile: the largest (128 x 128, BF16
@@ -1113,11 +1123,12 @@ struct GemmPlan {
   int tm, tn, ks, slices;
   int rb;  // the registers-B kernel (tm, tn, ks unused)
 };
+// What a K split of several weights may do: not be, leave its planes to the
+// caller, or be summed here.
+enum SplitMany { kSplitNone, kSplitLeft, kSplitSum };
 constexpr int kMaxSplitK = 8;
 
-// multi_split: a K split may take several weights (their planes are left to
-// the caller, not summed).
-GemmPlan plan_gemm(const g4_w4 *const *w, int nw, int rows, bool f32x, bool multi_split = false) {
+GemmPlan plan_gemm(const g4_w4 *const *w, int nw, int rows, bool f32x, SplitMany many = kSplitNone) {
   const int cus = cu_count() > 0 ? cu_count() : 256;
   if (w[0]->G % 2 != 0) return {2, 2, 1, 1};
   bool tiled = true;  // the packed-weight kernel reads every weight's tile copy
@@ -1130,18 +1141,24 @@ GemmPlan plan_gemm(const g4_w4 *const *w, int nw, int rows, bool f32x, bool mult
   };
   bool n96 = true;
   for (int i = 0; i < nw; ++i) n96 = n96 && w[i]->N % 96 == 0;
-  const int split_ok = nw == 1 || multi_split;  // summed K splits take one weight
+  const bool sum_many = nw > 1 && many == kSplitSum;
+  const bool split_ok = nw == 1 || many == kSplitLeft;
   {
     // registers-B tiles: 128 x 192 (BF16 x) or 64 x 192 (FP32 x), split K
     // into slices of at least 8 stages while that keeps the grid within two
     // blocks per CU
     const long b = blocks(f32x ? 64 : 128, 192);
     if (tiled && b >= cus) return {0, 0, 0, 1, 1};
-    if (tiled && split_ok) {
+    if (tiled && (split_ok || sum_many)) {
       int slices = 1;
       for (int k = 2; k <= kMaxSplitK; ++k)
         if (S % k == 0 && S / k >= 8 && b * k <= 2L * cus) slices = k;
-      if (b * slices >= cus) return {0, 0, 0, slices, 1};
+      if (split_ok && b * slices >= cus) return {0, 0, 0, slices, 1};
+      // several weights and their sum (q/k/v at K 1536, 389 rows: 33.6 -> 26.0
+      // us, 800: 39.6 -> 32.6), but not in place of whole rounds of 64 x 96
+      // tiles (gate and up of 6144, 100 rows: 24.1 us, 27.4 split)
+      if (sum_many && slices > 1 && b * slices >= cus - cus / 8 && !(n96 && blocks(64, 96) % cus == 0))
+        return {0, 0, 0, slices, 1};
     }
   }
   // FP32 x holds two planes of x' in LDS: 128-row tiles then fit one block
@@ -1227,13 +1244,24 @@ size_t part_bytes(const g4_w4 *const *w, int nw, int rows, int slices) {
   return slices > 1 ? slices * splitk_pstride(w, nw, rows) * 4 : 0;
 }
 
+// Whether several weights over rows x run as one launch with a summed K split:
+// where that is the plan and, in a recording, the scratch is there already.
+bool joint_split(const g4_w4 *const *w, int nw, int rows, bool f32x) {
+  const GemmPlan p = plan_gemm(w, nw, rows, f32x, kSplitSum);
+  if (!f32x || nw < 2 || !p.rb || p.slices < 2) return false;
+  int Mp;
+  size_t eoff, xend;
+  xprep_layout(w[0]->K, rows, f32x, &Mp, &eoff, &xend);
+  return !encoding() || g_ws.bytes >= ((xend + 255) & ~size_t(255)) + part_bytes(w, nw, rows, p.slices);
+}
+
 int gemm_scratch(const g4_w4 *const *w, int nw, bool f32x, int rows, bool prepped,
-                 GemmScratch *sc, const ExtScratch *ext, bool multi_split, bool sum, bool glu) {
+                 GemmScratch *sc, const ExtScratch *ext, SplitMany many, bool sum, bool glu) {
   const g4_w4 *w0 = w[0];
   size_t eoff, xend;
   xprep_layout(w0->K, rows, f32x, &sc->Mp, &eoff, &xend);
   const size_t poff = prepped ? 0 : (xend + 255) & ~size_t(255);
-  sc->plan = plan_gemm(w, nw, rows, f32x, multi_split);
+  sc->plan = plan_gemm(w, nw, rows, f32x, many);
   size_t need = poff + part_bytes(w, nw, rows, sc->plan.slices);
   // with x' prepared there is no pre-pass to save, only the wait per stage: the
   // engine's prompts (us saved per prompt of 37 / 128 / 301 / 512 tokens: 790 /
@@ -1257,15 +1285,16 @@ int gemm_scratch(const g4_w4 *const *w, int nw, bool f32x, int rows, bool preppe
     sc->part = reinterpret_cast<float *>(static_cast<char *>(ext->mem) + (sc->few ? 0 : poff));
     return G4_OK;
   }
-  if (sc->few && !prepped) {
-    // the scratch grows as it would for the prefill GEMM, so that what may be
-    // recorded after this call does not depend on the kernel it took; a
-    // recording needs the planes alone
-    for (int i = 0; i < nw && nw > 1; ++i) {
+  if (!prepped && !encoding()) {
+    // the scratch also has room for the weights one by one, and for the prefill
+    // GEMM of a few rows, so that what may be recorded after this call does not
+    // depend on the kernel it took
+    for (int i = 0; i < nw && nw > 1 && sum && !glu; ++i) {
       const size_t one = poff + part_bytes(w + i, 1, rows, plan_gemm(w + i, 1, rows, f32x).slices);
       if (one > need) need = one;
     }
-    if (encoding()) need = few;
+  } else if (!prepped && sc->few) {
+    need = few;  // a recording needs the planes alone
   }
   if (need > 0)
     if (int rc = g_ws.get(need, &ws, "g4_w4_linear (prefill)")) return rc;
@@ -1291,15 +1320,17 @@ static int gemm_run(const g4_w4 *const *w, int nw, const void *x, bool f32x, int
   long tiles64 = 0;
   for (int i = 0; i < nw; ++i) tiles64 += (long)((rows + 63) / 64) * ((w[i]->N + 63) / 64);
   GemmSmallPlan few;
-  if (nw > 1 && tiles64 < cus && !glu && x && !keep &&
-      !gemm_small_plan(w, nw, rows, false, true, &few)) {
+  const bool many = nw > 1 && !glu && x && !keep;
+  const bool sum_many = many && joint_split(w, nw, rows, f32x);
+  if (many && tiles64 < cus && !sum_many && !gemm_small_plan(w, nw, rows, false, true, &few)) {
     for (int i = 0; i < nw; ++i)
       if (int rc = gemm_run(w + i, 1, x, f32x, rows, y + i, y_bf16, nullptr)) return rc;
     return G4_OK;
   }
   const g4_w4 *w0 = w[0];
   GemmScratch sc;
-  if (int rc = gemm_scratch(w, nw, f32x, rows, !x, &sc, ext, keep && nw > 1, !keep, glu)) return rc;
+  if (int rc = gemm_scratch(w, nw, f32x, rows, !x, &sc, ext,
+                            keep && nw > 1 ? kSplitLeft : sum_many ? kSplitSum : kSplitNone, !keep, glu)) return rc;
   const GemmPlan plan = sc.plan;
   const int Mp = sc.Mp;
   uint4 *xt = sc.xt;
@@ -1322,7 +1353,7 @@ static int gemm_run(const g4_w4 *const *w, int nw, const void *x, bool f32x, int
                                    glu))
       return rc;
     return slices > 1 && sum
-               ? launch_splitk_sum(part, slices, pstride, (size_t)rows * w0->N, y[0], y_bf16)
+               ? launch_splitk_sum(part, slices, w, nw, rows, y, y_bf16)
                : G4_OK;
   }
   if (!x)
@@ -1421,8 +1452,7 @@ int w4_gemm_few(const g4_w4 *w, const void *x, int rows, void *y, bool y_bf16,
   if (int rc = launch_gemm_small(p, &w, 1, x, true, nullptr, nullptr, 0, rows, &y, y_bf16, part,
                                  pstride, false))
     return rc;
-  return p.slices > 1 ? launch_splitk_sum(part, p.slices, pstride, (size_t)rows * w->N, y, y_bf16)
-                      : G4_OK;
+  return p.slices > 1 ? launch_splitk_sum(part, p.slices, &w, 1, rows, &y, y_bf16) : G4_OK;
 }
 
 bool w4_gemm_few_joint(const g4_w4 *const *w, int nw, int rows) {

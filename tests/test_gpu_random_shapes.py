@@ -129,6 +129,35 @@ def test_few_rows_several_weights_and_recorded(g4, rows, k, widths):
             np.testing.assert_array_equal(y.download(np.float32), w)
 
 
+@pytest.mark.parametrize("rows,widths", [(290, (2048, 256, 256)), (389, (2047, 250, 33)),
+                                         (640, (1536, 640)), (1000, (600, 1001))])
+@pytest.mark.parametrize("bf16_out", [False, True])
+def test_several_weights_with_a_summed_split(g4, rows, widths, bf16_out):
+    # joint launches whose K split is summed into each weight's output, at row
+    # counts and widths whose products are and are not multiples of four
+    k = 1536
+    rng = np.random.default_rng([rows, len(widths)])
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    xb = g4.Buffer.from_array(x)
+    lins, refs = [], []
+    for n in widths:
+        packed, scales, q = syn.w4_weights(n, n, k)
+        lins.append(g4.W4Linear(packed, scales))
+        refs.append(x.astype(np.float64) @ dense(q, scales).T)
+    size = 2 if bf16_out else 4
+    ys = [g4.Buffer(rows * n * size) for n in widths]
+    g4.W4Linear.linear_multi(lins, xb.ptr, g4.F32, rows, [y.ptr for y in ys],
+                             g4.BF16 if bf16_out else g4.F32)
+    for y, n, ref in zip(ys, widths, refs):
+        if bf16_out:
+            got = syn.bf16_to_f32(y.download(np.uint16)).reshape(rows, n)
+        else:
+            got = y.download(np.float32).reshape(rows, n)
+        # 22-bit x and FP32 sums; BF16 has 8 significant bits: half an ulp is at
+        # most 2^-8 of each value
+        assert rel_l2_rows(got, ref) <= 2e-6 + (2.0 ** -8 if bf16_out else 0)
+
+
 @pytest.mark.parametrize("k", [16384, 32768])
 @pytest.mark.parametrize("rows", [1, 3, 40])
 @pytest.mark.parametrize("f32x", [False, True])
