@@ -15,6 +15,7 @@
 
 #include <vector>
 
+#include "g4_gemv.h"
 #include "g4_internal.h"
 #include "g4_ops.h"
 
@@ -72,15 +73,7 @@ __global__ __launch_bounds__(1024) void advance_kernel(const float2 *__restrict_
       }
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
-    if (ov > bv || (ov == bv && oi < bi)) {
-      bv = ov;
-      bi = oi;
-    }
-  }
+  wave_argmax(bv, bi);
   if ((threadIdx.x & 63) == 0) {
     sv[threadIdx.x >> 6] = bv;
     si[threadIdx.x >> 6] = bi;

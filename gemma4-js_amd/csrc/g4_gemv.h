@@ -72,6 +72,33 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (r0 + r1) + (r2 + r3);
 }
 
+// The largest value of a wave and, among its holders, the smallest index, in
+// every lane (lane swaps and DPP moves: shuffles take a trip through LDS each).
+// v is no NaN.
+__device__ __forceinline__ void wave_argmax(float &v, int &i) {
+  const auto up = [](float a, float b) { return fmaxf(a, b); };
+  float m = v;
+  m = up(m, dpp_f32<0xB1>(m));   // quad_perm [1,0,3,2]
+  m = up(m, dpp_f32<0x4E>(m));   // quad_perm [2,3,0,1]
+  m = up(m, dpp_f32<0x141>(m));  // row_half_mirror
+  m = up(m, dpp_f32<0x140>(m));  // row_mirror
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  m = up(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  a = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  m = up(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  int x = v == m ? i : 0x7fffffff;
+  const auto low = [](int p, int q) { return p < q ? p : q; };
+  x = low(x, __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, true));
+  x = low(x, __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, true));
+  x = low(x, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true));
+  x = low(x, __builtin_amdgcn_update_dpp(0, x, 0x140, 0xf, 0xf, true));
+  a = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+  x = low((int)a[0], (int)a[1]);
+  a = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+  v = m;
+  i = low((int)a[0], (int)a[1]);
+}
+
 __device__ __forceinline__ uint32_t bf16_pair(uint32_t lo16, uint32_t hi16) {
   return (lo16 & 0xffffu) | (hi16 << 16);
 }

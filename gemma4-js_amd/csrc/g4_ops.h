@@ -124,6 +124,6 @@ int launch_bf16_head(const float *x, const uint16_t *E, int rows, int K, float *
                      float softcap, float2 *partials);
 int launch_argmax_partials(const float2 *partials, int nparts, int *out_idx);
 int launch_argmax(const float *x, int n, float2 *partials, int *out_idx);
-size_t argmax_blocks(int n);
+size_t argmax_partials();  // launch_argmax's, whatever n
 
 }  // namespace g4

@@ -1622,7 +1622,7 @@ G4_API int g4_argmax(const float *x, int n, int32_t *out_dev) {
   int rc = check_f32(x, n, "g4_argmax x");
   if (!rc) rc = check_device_range(out_dev, 4, "g4_argmax out");
   void *part = nullptr;
-  if (!rc) rc = g_argmax_ws.get(argmax_blocks(n) * sizeof(float2), &part, "g4_argmax");
+  if (!rc) rc = g_argmax_ws.get(argmax_partials() * sizeof(float2), &part, "g4_argmax");
   if (!rc) rc = launch_argmax(x, n, static_cast<float2 *>(part), out_dev);
   return rc ? rc : ok();
 }

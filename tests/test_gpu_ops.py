@@ -422,6 +422,20 @@ def test_argmax_first_index_of_max_skipping_nonfinite(g4, oracle, n):
     assert got == int(oracle.topk(x, 1)[0][0])
 
 
+@pytest.mark.parametrize("n", [1023, 1025, 262144, (1 << 20) + 1, 1300000])
+def test_argmax_blocks_of_1024_and_more(g4, n):
+    # one round of four loads per thread, several rounds past 2^20 values, and
+    # the first of equal maxima in any lane, wave and block
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n).astype(np.float32)
+    x[rng.integers(0, n, 7)] = np.inf
+    for at in sorted(rng.integers(0, n, 9).tolist() + [n - 1], reverse=True):
+        x[at] = 9.5
+        o = out(g4, 1, np.int32)
+        g4.argmax(dev(g4, x), n, o)
+        assert int(o.download(np.int32)[0]) == at
+
+
 def test_argmax_no_finite_value(g4):
     x = np.array([np.nan, np.inf, -np.inf], np.float32)
     o = out(g4, 1, np.int32)
