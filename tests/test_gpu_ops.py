@@ -436,6 +436,24 @@ def test_argmax_blocks_of_1024_and_more(g4, n):
         assert int(o.download(np.int32)[0]) == at
 
 
+@pytest.mark.parametrize("heads", [4, 8])
+@pytest.mark.parametrize("hd,angles", [(256, 128), (512, 64)])
+def test_norm_rope_many_heads_equal_one_row_calls(g4, heads, hd, angles):
+    # four heads per wave against one block per head: the same bits
+    rows = 2048 // heads + 5
+    rng = np.random.default_rng([heads, hd])
+    x = rng.standard_normal((rows, heads * hd)).astype(np.float32)
+    w = rng.standard_normal(hd).astype(np.float32)
+    wb = dev(g4, w)
+    y = out(g4, x.size)
+    g4.norm_rope(dev(g4, x), rows, heads, hd, 37, wb, angles, 10000.0, y)
+    got = y.download(np.float32).reshape(x.shape)
+    one = out(g4, heads * hd)
+    for r in (0, 1, 63, rows - 2, rows - 1):
+        g4.norm_rope(dev(g4, x[r]), 1, heads, hd, 37 + r, wb, angles, 10000.0, one)
+        np.testing.assert_array_equal(got[r], one.download(np.float32))
+
+
 def test_argmax_no_finite_value(g4):
     x = np.array([np.nan, np.inf, -np.inf], np.float32)
     o = out(g4, 1, np.int32)
