@@ -23,13 +23,13 @@
 //
 // Measured (us per call, 8 heads, against the FP32 matrix kernels in
 // g4_ops.hip on one box; error against binary64 in parentheses):
-//   head dim 512, all keys   2048 rows, 4096 keys   1387 (8.0e-7) -> 622 (4.1e-7)
-//                            1500 rows, 3000 keys    785 (7.1e-7) -> 464 (3.8e-7)
+//   head dim 512, all keys   2048 rows, 4096 keys   1387 (8.0e-7) -> 580 (4.1e-7)
+//                            1500 rows, 3000 keys    785 (7.1e-7) -> 374 (3.8e-7)
 //                            20 rows, 2020 keys      216 -> 40
 //                            512 rows, 512 keys       61 (3.0e-7) -> 49 (2.3e-7)
 //   head dim 256, window 512 1500 rows, 3000 keys    103 (4.8e-7) -> 70 (3.0e-7)
 //                            20 rows, 2020 keys       35 -> 24
-// The long case is 170 TFLOP/s in FP32 terms.  Its block step of 32 keys takes
+// The long case is 180 TFLOP/s in FP32 terms.  Its block step of 32 keys takes
 // about 5 us against 2 us of matrix work: with the loads left out it was 70% of
 // the time, with the score products left out 59%, with softmax and barriers
 // alone 30%.
@@ -778,6 +778,10 @@ struct RowsPlan {
   size_t kv, meta, part, total;  // floats
 };
 
+constexpr int kMaxKeys = 16384;  // launch_attention's limit
+constexpr int kRing = 2048;
+static_assert(2 * (kMaxKeys / kTile + 1) + 4 < kRing, "a block's time fits the ring");
+
 int cus() { return cu_count() > 0 ? cu_count() : 256; }
 
 // Most keys that the rows of `positions` consecutive positions see.
@@ -786,9 +790,18 @@ int keys_seen(int positions, int max_keylen, bool sliding, int window) {
   return sliding && n < max_keylen ? (int)n : max_keylen;
 }
 
-// Key tiles of the call, and the split of a row block's tiles over blocks:
-// as many as fill the CUs (one block per CU at head dim 512, two below), at
-// least two tiles each, and no more than `avail` floats of scratch hold.
+// Key tiles of the call, and the split of a row block's tiles over blocks (at
+// least two tiles each, and no more than `avail` floats of scratch).
+// Head dim 256: as many as fill the CUs with two blocks each.
+// Head dim 512, one block per CU: the split whose blocks, dealt to the CUs in
+// launch order, end first by these measured costs in halves of a tile's 4.4 us:
+// 2 per tile, 4 per block (q's conversion, the first loads, the stores), 1 for a
+// block with no tiles (early rows have fewer than late ones, yet every block
+// needs its LDS), and with more than one split 3 for the merge and 1 per 36
+// blocks for its planes.  us per call at 8 heads by splits (* as chosen): 1000
+// rows over 1000 keys 175, 111, 88 *, 117; 700 over 2700 keys 419, 238, 175 *,
+// 247; 1500 over 1500 keys 247, 155 *, 197; 2048 over 4096 keys 623, 657, 611,
+// 580 *, 582, 626.
 bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int window,
                size_t avail, RowsPlan *p) {
   const int nrows = qrows * heads, blocks = cdiv(nrows, kRows);
@@ -799,20 +812,71 @@ bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int w
     return n < all ? n : all;
   };
   p->tiles = tiles_of(qrows);
-  const int nt = tiles_of(span < qrows ? span : qrows);
-  int splits = (hd > 256 ? 1 : 2) * cus() / blocks;
-  if (splits > kMaxSplits) splits = kMaxSplits;
   p->kv = (size_t)p->tiles * hd * 80;
   p->meta = (size_t)p->tiles * kMetaInts;
-  for (;; --splits) {
-    p->tps = splits > 1 ? cdiv(nt, splits) : nt;
-    if (p->tps < 2) p->tps = 2;
-    p->splits = cdiv(nt, p->tps);
-    p->part = p->splits > 1 ? (size_t)p->splits * nrows * (hd + 2) : 0;
+  const int nt = tiles_of(span < qrows ? span : qrows);
+  const int slots = cus();
+  // tiles of row block b (launched last to first), as the kernel counts them
+  const int qpos0 = max_keylen - qrows;
+  auto block_tiles = [&](int b) {
+    const int first = qpos0 + b * kRows / heads;
+    const int last = qpos0 + ((b + 1) * kRows < nrows ? (b + 1) * kRows - 1 : nrows - 1) / heads;
+    const int lo = sliding && first - window + 1 > 0 ? first - window + 1 : 0;
+    return last / kTile - lo / kTile + 1;
+  };
+  auto fits = [&](int splits) {
+    p->splits = splits;
+    p->part = splits > 1 ? (size_t)splits * nrows * (hd + 2) : 0;
     p->total = p->kv + p->meta + p->part;
-    if (p->total <= avail) return true;
-    if (splits <= 1) return false;
+    return p->total <= avail;
+  };
+  auto tiles_per = [&](int splits) {
+    const int t = cdiv(nt, splits);
+    return splits == 1 || t > 2 ? t : 2;
+  };
+  if (hd <= 256) {
+    int want = 2 * slots / blocks;
+    want = want > kMaxSplits ? kMaxSplits : want < 1 ? 1 : want;
+    for (; want >= 1; --want) {
+      p->tps = tiles_per(want);
+      if (fits(cdiv(nt, p->tps))) return true;
+    }
+    return false;
   }
+  // CUs that become free at each time, from `now` on (a block takes less than a
+  // turn of the ring: see kMaxKeys)
+  int free_at[kRing];
+  long best = -1;
+  int best_splits = 0, best_tps = 0, last_tps = 0;
+  for (int want = 1; want <= kMaxSplits; want += want < 6 ? 1 : want / 3) {
+    const int tps = tiles_per(want), splits = cdiv(nt, tps);
+    if (tps == last_tps) continue;
+    if (splits > 1 && (long)splits * blocks > 4L * slots) break;
+    last_tps = tps;
+    if (!fits(splits)) continue;
+    for (int &f : free_at) f = 0;
+    free_at[0] = slots;
+    long end = 0, used = 0, now = 0;
+    for (int y = 0; y < splits; ++y)
+      for (int b = blocks - 1; b >= 0; --b) {
+        int t = block_tiles(b) - y * tps;
+        t = t < tps ? t : tps;
+        const int len = t > 0 ? 2 * t + 4 : 1;
+        used += t > 0;
+        while (free_at[now % kRing] == 0) ++now;
+        --free_at[now % kRing];
+        ++free_at[(now + len) % kRing];
+        if (now + len > end) end = now + len;
+      }
+    if (splits > 1) end += 3 + used / 36;
+    if (best < 0 || end < best) {
+      best = end;
+      best_splits = splits;
+      best_tps = tps;
+    }
+  }
+  p->tps = best_tps;
+  return best >= 0 && fits(best_splits);
 }
 
 template <int HD>
@@ -845,7 +909,7 @@ int launch_rows(const RowsArgs &a, const RowsPlan &p) {
 // 256 keys 35 / 39; head dim 256, 20 rows over 220 keys 21 / 23, 370 keys 27 / 24,
 // 512 rows over 512 keys 33 / 39, 700 rows over 700 keys 51 / 45.
 bool attention_rows_wins(int qrows, int heads, int hd, int max_keylen, bool sliding, int window) {
-  if (hd != 256 && hd != 512) return false;
+  if ((hd != 256 && hd != 512) || max_keylen > kMaxKeys) return false;
   const int nrows = qrows * heads;
   const int keys = keys_seen(cdiv(16, heads) + 1, max_keylen, sliding, window);
   const int steps = cdiv(keys, 16) * cdiv(nrows, 16 * cus());
@@ -854,7 +918,7 @@ bool attention_rows_wins(int qrows, int heads, int hd, int max_keylen, bool slid
 
 size_t attention_rows_floats(int qrows, int heads, int hd, int max_keylen, bool sliding,
                              int window) {
-  RowsPlan p;
+  RowsPlan p{};
   if (!attention_rows_wins(qrows, heads, hd, max_keylen, sliding, window)) return 0;
   rows_plan(qrows, heads, hd, max_keylen, sliding, window, ~size_t(0), &p);
   return p.total;
@@ -864,7 +928,7 @@ int launch_attention_rows(const float *q, const float *k, const float *v, int qr
                           int hd, int keylen, int qpos0, const int *pos_dev, int max_keylen,
                           bool sliding, int window, float *scratch, size_t scratch_floats,
                           float *out, void *xt, int *xe, int Mp, bool *taken) {
-  RowsPlan p;
+  RowsPlan p{};
   *taken = false;
   if (!rows_plan(qrows, heads, hd, max_keylen, sliding, window, scratch_floats, &p)) return G4_OK;
   RowsArgs a{};

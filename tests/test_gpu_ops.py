@@ -275,7 +275,7 @@ def run_attention(g4, q, k, v, qrows, heads, hd, keylen, qpos0, sliding, window)
     (9, 8, 512, 1000, 0, True, 333), (33, 8, 512, 545, 32, False, 0), (40, 5, 512, 290, 0, True, 511),
     (2, 8, 256, 353, 0, False, 0), (3, 7, 256, 900, 65, True, 512), (17, 8, 256, 416, 0, False, 0),
     (64, 4, 256, 1057, 0, True, 500), (700, 8, 256, 700, 0, True, 512), (513, 8, 512, 513, 0, True, 300),
-    (1100, 8, 256, 1100, 0, False, 0),
+    (1100, 8, 256, 1100, 0, False, 0), (260, 8, 512, 900, 0, False, 0), (90, 8, 512, 2100, 3, False, 0),
 ])
 def test_attention_rows_over_long_caches(g4, qrows, heads, hd, keylen, tail, sliding, window):
     q, k, v, qpos0 = rows_case(qrows, heads, hd, keylen, tail, 21)
