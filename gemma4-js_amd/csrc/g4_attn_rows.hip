@@ -22,7 +22,7 @@
 //   attn_rows_merge_kernel  adds the key splits
 //
 // Measured (us per call, 8 heads, against the FP32 matrix kernels in
-// g4_ops.hip on one box; error against binary64 in parentheses):
+// g4_ops.hip; error against binary64 in parentheses):
 //   head dim 512, all keys   2048 rows, 4096 keys   1387 (8.0e-7) -> 580 (4.1e-7)
 //                            1500 rows, 3000 keys    785 (7.1e-7) -> 374 (3.8e-7)
 //                            20 rows, 2020 keys      216 -> 40
