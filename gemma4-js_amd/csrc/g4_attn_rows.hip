@@ -23,13 +23,13 @@
 //
 // Measured (us per call, 8 heads, against the FP32 matrix kernels in
 // g4_ops.hip; error against binary64 in parentheses):
-//   head dim 512, all keys   2048 rows, 4096 keys   1387 (8.0e-7) -> 580 (4.1e-7)
+//   head dim 512, all keys   2048 rows, 4096 keys   1387 (8.0e-7) -> 572 (3.8e-7)
 //                            1500 rows, 3000 keys    785 (7.1e-7) -> 374 (3.8e-7)
 //                            20 rows, 2020 keys      216 -> 40
-//                            512 rows, 512 keys       61 (3.0e-7) -> 49 (2.3e-7)
-//   head dim 256, window 512 1500 rows, 3000 keys    103 (4.8e-7) -> 70 (3.0e-7)
+//                            512 rows, 512 keys       61 (3.0e-7) -> 51 (2.3e-7)
+//   head dim 256, window 512 1500 rows, 3000 keys    103 (4.8e-7) -> 74 (3.0e-7)
 //                            20 rows, 2020 keys       35 -> 24
-// The long case is 180 TFLOP/s in FP32 terms.  Its block step of 32 keys takes
+// The long case is 181 TFLOP/s in FP32 terms.  Its block step of 32 keys takes
 // about 5 us against 2 us of matrix work: with the loads left out it was 70% of
 // the time, with the score products left out 59%, with softmax and barriers
 // alone 30%.
@@ -430,8 +430,11 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
     f16x8 ph, pl;
     float p[8], s[8], osc = 0.f;
     bool slow = false;
-    // the scores of 16 keys over this wave's dims: the leading products in
-    // sums of 128 dims; the pieces of two steps are read ahead
+    // the scores of 16 keys over this wave's dims: the leading products in sums
+    // of 128 dims.  The order of reads and products is the compiler's, and the
+    // wave goes first on its SIMD meanwhile (1500 rows over 3000 keys: 384 us
+    // with one step's pieces read ahead by scheduling groups, 375 so; for the
+    // outputs below the groups are worth 583 against 657 us at 2048 over 4096)
     auto scores = [&](const u32x4 *buf, float *sc) {
       const u32x4 *kb = buf + dh * (NJ * 3 * 64) + lane;
       constexpr int NM = NJ > 4 ? NJ / 4 : 1;
@@ -454,25 +457,24 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
         d2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][1], qp[j][1], d2, 0, 0, 0);
         d3 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[j][2], qp[j][0], d3, 0, 0, 0);
       }
-      constexpr int AHEAD = 1;
-      __builtin_amdgcn_sched_group_barrier(0x100, 3 * AHEAD, 0);
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
-        if (j + AHEAD < NJ) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-      }
       f32x4 d = d1 + (d2 + d3);
 #pragma unroll
       for (int i = 0; i < NM; ++i) d += d0[i];
 #pragma unroll
       for (int v = 0; v < 4; ++v) sc[v] = d[v];
     };
-    if (mine) scores(sm.a, s);
+    if (mine) {
+      __builtin_amdgcn_s_setprio(1);
+      scores(sm.a, s);
+      __builtin_amdgcn_s_setprio(0);
+    }
     // B has landed everywhere, and A is free
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (kt < t1) load_k(kt + 1, 0);
     if (mine) {
+      __builtin_amdgcn_s_setprio(1);
       scores(sm.b, s + 4);
+      __builtin_amdgcn_s_setprio(0);
       if (DH > 1) {
         sm.ex[w][0][lane] = (f32x4){s[0], s[1], s[2], s[3]};
         sm.ex[w][1][lane] = (f32x4){s[4], s[5], s[6], s[7]};
