@@ -145,8 +145,9 @@ struct g4_w4 {
 };
 
 namespace g4 {
-// Activation rows up to which g4_w4_linear streams the weights (GEMV); more
-// rows take the MFMA GEMM.
+// Activation rows up to which g4_w4_linear may stream the weights (GEMV; FP32
+// rows 2 to 4 only where w4_gemm_few leaves them); more rows take the matrix
+// cores.
 constexpr int kMaxGemvRows = 4;
 // Prefill GEMM (more than kMaxGemvRows rows): y[rows, N] = x[rows, K] . W^T on
 // the matrix cores (g4_gemm.hip).
