@@ -3,36 +3,34 @@
 // matrix cores.
 //
 // Numerics.  The 16-bit matrix forms run at 16 times the FP32 form's rate, so
-// FP32 operands are split and the sums stay in FP32.
-//   scores   q and k as three BF16 parts each (exact: 3 x 8 bits), six
-//            v_mfma_f32_16x16x32_bf16; the dropped products are below 2^-26.
-//            An error of a score is a relative error of its probability, and
-//            two FP16 parts (22 bits, three products) left 1.3-1.7 times the
-//            FP32 form's error at head dim 512.
-//   outputs  v and p as two FP16 parts 2^e (hi + lo), three
-//            v_mfma_f32_16x16x32_f16 (hi.hi, hi.lo, lo.hi).  v has one
-//            exponent per key, folded into that key's probability; p has one
-//            per query row and key tile (that of the tile's largest p 2^e_v),
-//            so no range of values is out of reach.
+// q, k, v and p are taken as three BF16 parts each (exact: 3 x 8 bits of FP32's
+// 24, and FP32's exponents), six v_mfma_f32_16x16x32_bf16 per product, the sums
+// in FP32.  What is dropped is below 2^-26 of each product by itself, so a small
+// value keeps its bits beside any large one (below 2^-110 the last parts leave
+// BF16's range).  Two FP16 parts under shared
+// exponents were less: for the scores 1.3-1.7 times the FP32 form's error at head
+// dim 512, and a value 1e-8 of the largest of its key lost half of its bits.
 //
 // Two launches, three where the keys are split over blocks:
-//   attn_kv_split_kernel    k and v of the visible keys as FP16 hi/lo in the
-//                           order the matrix instructions read them
-//   attn_rows_f16_kernel    64 rows of [qrows * heads, hd] per block
+//   attn_kv_split_kernel    the parts of k and v of the visible keys in the order
+//                           the matrix instructions read them
+//   attn_rows_split_kernel  64 rows of [qrows * heads, hd] per block
 //   attn_rows_merge_kernel  adds the key splits
 //
 // Measured (us per call, 8 heads, against the FP32 matrix kernels in
 // g4_ops.hip; error against binary64 in parentheses):
-//   head dim 512, all keys   2048 rows, 4096 keys   1387 (8.0e-7) -> 572 (3.8e-7)
-//                            1500 rows, 3000 keys    785 (7.1e-7) -> 374 (3.8e-7)
-//                            20 rows, 2020 keys      216 -> 40
-//                            512 rows, 512 keys       61 (3.0e-7) -> 51 (2.3e-7)
-//   head dim 256, window 512 1500 rows, 3000 keys    103 (4.8e-7) -> 74 (3.0e-7)
-//                            20 rows, 2020 keys       35 -> 24
-// The long case is 181 TFLOP/s in FP32 terms.  Its block step of 32 keys takes
-// about 5 us against 2 us of matrix work: with the loads left out it was 70% of
-// the time, with the score products left out 59%, with softmax and barriers
-// alone 30%.
+//   head dim 512, all keys   2048 rows, 4096 keys   1384 (8.0e-7) -> 670 (3.7e-7)
+//                            1500 rows, 3000 keys    784 (7.1e-7) -> 431 (3.6e-7)
+//                            1000 rows, 1000 keys    171 (3.7e-7) -> 101 (2.5e-7)
+//                            20 rows, 2020 keys      213 (6.5e-7) -> 40 (3.7e-7)
+//                            512 rows, 512 keys       62 (3.0e-7) -> 55 (2.2e-7)
+//   head dim 256, window 512 1500 rows, 3000 keys    106 (4.8e-7) -> 77 (3.0e-7)
+//                            20 rows, 2020 keys       34 (5.0e-7) -> 23 (2.9e-7)
+// The long case is 154 TFLOP/s in FP32 terms.  Its block step of 32 keys takes
+// about 5.2 us against 2.7 us of matrix work: with the tile loads left out the
+// call takes 82% of its time, without the score products 67%, without the output
+// products 78%, with softmax and barriers alone 25%.  (v and p as two FP16 parts,
+// three products, took 568 us there and 365 over 3000 keys.)
 #include <math.h>
 
 #include <type_traits>
@@ -52,9 +50,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 constexpr int kTile = 32;      // keys per tile
 constexpr int kRows = 64;      // query rows (of qrows * heads) per block
 constexpr int kMaxSplits = 64;  // key splits of one call
-// Per tile: [0, 32) 2^(e_v - max e_v) of each key, 32 max e_v, 33 and 34 the
-// flags of K and V.
-constexpr int kMetaInts = 64;
+constexpr int kTileFlags = 2;  // per tile: K's and V's
 
 struct RowsArgs {
   const float *q, *k, *v;
@@ -62,8 +58,8 @@ struct RowsArgs {
   uint4 *xt;  // the prefill GEMM's x' (w4_gemm_prepare), instead of out
   int *xe;
   int Mp;
-  u32x4 *kv;   // split tiles: 32 hd 6 bytes of K, then 32 hd 4 of V
-  int *meta;   // per tile kMetaInts
+  u32x4 *kv;   // split tiles: 32 hd 6 bytes of K, then of V
+  int *flags;  // per tile kTileFlags
   float *part;  // [splits][nrows][hd] unnormalised outputs
   float2 *ml;   // [splits][nrows] (max, sum)
   int H, hd, keylen, qpos0, sliding, window, qrows;
@@ -104,11 +100,6 @@ __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[3]) {
   }
 }
 
-// Exponent that brings a row of largest magnitude mx (as bits) to [2^13, 2^14).
-__device__ __forceinline__ int row_exp(uint32_t mx) {
-  return __builtin_amdgcn_frexp_expf(__uint_as_float(mx)) - 14;
-}
-
 // max over the lanes c, c + 16, c + 32, c + 48
 __device__ __forceinline__ float group_max(float v) {
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -118,9 +109,7 @@ __device__ __forceinline__ float group_max(float v) {
 }
 
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr uint32_t kInfBits = 0x7f800000u;
 constexpr uint32_t kBf16MaxBits = 0x7f7f8000u;  // from here on BF16 rounds to infinity
-constexpr int kZeroExp = -200;  // e_v of an all-zero row: its probability becomes 0
 
 // Waves that share a row's head dim (its q and output dims), and the place of
 // V piece n: first the first halves of every such wave's dims.
@@ -133,33 +122,40 @@ __device__ constexpr int v_piece(int n) {
   return (i / (NW / 2)) * (NN / 2) + dh * (NW / 2) + i % (NW / 2);
 }
 
-// K (blockIdx.y 0) or V (1) of one 32-key tile.  K piece (sub, j) is the A
-// operand of score step j for keys 16 sub ..: lane (c, g) holds key c, dims
-// 32 j + 8 g .. + 7, three parts of 1 KB.  V piece n is the A operand of output
-// dims 16 n ..: lane (c, g) holds dim 16 n + c of keys 4 g .. + 3 and 16 + 4 g
-// .. + 3, the keys whose probabilities lane group g computes, 1 KB of hi and
-// 1 KB of lo.  Rows past the last visible key are zeros and are not read.  A
-// row with a non-finite value is stored as zeros and flags its tile, which
-// the attention kernel then computes from the FP32 rows.  Bound by the
-// latency of its loads and of the reduction behind them.
+// K (blockIdx.y 0) or V (1) of one 32-key tile, three parts of 1 KB per piece.
+// K piece (sub, j) is the A operand of score step j for keys 16 sub ..: lane
+// (c, g) holds key c, dims 32 j + 8 g .. + 7.  V piece n is the A operand of
+// output dims 16 n ..: lane (c, g) holds dim 16 n + c of keys 4 g .. + 3 and
+// 16 + 4 g .. + 3, the keys whose probabilities lane group g computes.  Rows
+// past the last visible key are zeros and are not read.  A value that BF16
+// parts cannot hold (not finite, or within 2^-9 of FP32's largest) flags its
+// tile, which the attention kernel then computes from the FP32 rows.  Bound by
+// the latency of its loads.
 template <int HD>
 __global__ __launch_bounds__(512) void attn_kv_split_kernel(RowsArgs a) {
   constexpr int KI = (HD / 32 + 3) / 4, VI = (HD / 16 + 7) / 8;
-  __shared__ uint32_t mxs[8][32];
-  __shared__ int flag;
   const Span sp(a);
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, c = lane & 15, g = lane >> 4;
   const int slot = blockIdx.x, k0 = (sp.base(a) + slot) * kTile;
   const int kmax = sp.kmax(sp.qpos0 + a.qrows - 1);
   if (k0 > kmax) return;
-  u32x4 *dst = a.kv + (size_t)slot * (20 * HD) + (blockIdx.y ? 12 * HD : 0);
-  int *meta = a.meta + (size_t)slot * kMetaInts;
-  if (t == 0) flag = 0;
+  u32x4 *dst = a.kv + (size_t)slot * (24 * HD) + (blockIdx.y ? 12 * HD : 0);
+  uint32_t mx = 0;
+  auto store = [&](const float (&x)[8], int piece) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t b = __float_as_uint(x[e]) & 0x7fffffffu;
+      mx = b > mx ? b : mx;
+    }
+    bf16x8 p[3];
+    split8(x, p);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) dst[(piece * 3 + q) * 64 + lane] = __builtin_bit_cast(u32x4, p[q]);
+  };
   if (blockIdx.y == 0) {
     const int sub = w & 1, key = k0 + 16 * sub + c;
     const float *src = a.k + (size_t)(key <= kmax ? key : kmax) * HD + 8 * g;
     float x[KI][8];
-    uint32_t mx = 0;
 #pragma unroll
     for (int i = 0; i < KI; ++i) {
       const int j = (w >> 1) + 4 * i;
@@ -167,44 +163,15 @@ __global__ __launch_bounds__(512) void attn_kv_split_kernel(RowsArgs a) {
       const float4 u0 = p[0], u1 = p[1];
       const float y[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[i][e] = key <= kmax ? y[e] : 0.f;
-        const uint32_t b = __float_as_uint(x[i][e]) & 0x7fffffffu;
-        mx = b > mx ? b : mx;
-      }
+      for (int e = 0; e < 8; ++e) x[i][e] = key <= kmax ? y[e] : 0.f;
     }
-#pragma unroll
-    for (int o = 16; o <= 32; o <<= 1) {
-      const uint32_t b = __shfl_xor(mx, o, 64);
-      mx = b > mx ? b : mx;
-    }
-    if (g == 0) mxs[w][c] = mx;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t b = mxs[2 * i + sub][c];
-      mx = b > mx ? b : mx;
-    }
-    const bool bad = mx >= kBf16MaxBits;
-    if (bad) flag = 1;
 #pragma unroll
     for (int i = 0; i < KI; ++i) {
       const int j = (w >> 1) + 4 * i;
-      if (j >= HD / 32) continue;
-      if (bad)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) x[i][q] = 0.f;
-      bf16x8 p[3];
-      split8(x[i], p);
-#pragma unroll
-      for (int q = 0; q < 3; ++q)
-        dst[((sub * (HD / 32) + j) * 3 + q) * 64 + lane] = __builtin_bit_cast(u32x4, p[q]);
+      if (j < HD / 32) store(x[i], sub * (HD / 32) + j);
     }
-    __syncthreads();
-    if (t == 0) meta[33] = flag;
   } else {
     float x[VI][8];
-    uint32_t mx[8] = {};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int key = k0 + (e < 4 ? 4 * g + e : 12 + 4 * g + e);
@@ -214,66 +181,16 @@ __global__ __launch_bounds__(512) void attn_kv_split_kernel(RowsArgs a) {
         const int n = w + 8 * i;
         const float y = src[16 * (n < HD / 16 ? n : 0)];
         x[i][e] = key <= kmax ? y : 0.f;
-        const uint32_t b = __float_as_uint(x[i][e]) & 0x7fffffffu;
-        mx[e] = b > mx[e] ? b : mx[e];
       }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-#pragma unroll
-      for (int o = 1; o <= 8; o <<= 1) {
-        const uint32_t b = __shfl_xor(mx[e], o, 64);
-        mx[e] = b > mx[e] ? b : mx[e];
-      }
-      if (c == 0) mxs[w][8 * g + e] = mx[e];
-    }
-    __syncthreads();
-    int ev[8];
-    bool bad[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      uint32_t m = 0;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t b = mxs[i][8 * g + e];
-        m = b > m ? b : m;
-      }
-      bad[e] = m >= kInfBits;
-      ev[e] = bad[e] || m == 0 ? kZeroExp : row_exp(m);
-      if (bad[e]) flag = 1;
-    }
-    int em = ev[0];
-#pragma unroll
-    for (int e = 1; e < 8; ++e) em = ev[e] > em ? ev[e] : em;
-#pragma unroll
-    for (int o = 16; o <= 32; o <<= 1) {
-      const int b = __shfl_xor(em, o, 64);
-      em = b > em ? b : em;
-    }
-    if (w == 0 && c == 0) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        meta[e < 4 ? 4 * g + e : 12 + 4 * g + e] = __float_as_int(ldexpf(1.f, ev[e] - em));
-      if (g == 0) meta[32] = em;
     }
 #pragma unroll
     for (int i = 0; i < VI; ++i) {
       const int n = w + 8 * i;
-      if (n >= HD / 16) continue;
-      f16x8 hi, lo;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float s = bad[e] ? 0.f : ldexpf(x[i][e], -ev[e]);
-        hi[e] = (_Float16)s;
-        lo[e] = (_Float16)(s - (float)hi[e]);
-      }
-      const int at = v_piece<HD>(n);
-      dst[(2 * at) * 64 + lane] = __builtin_bit_cast(u32x4, hi);
-      dst[(2 * at + 1) * 64 + lane] = __builtin_bit_cast(u32x4, lo);
+      if (n < HD / 16) store(x[i], v_piece<HD>(n));
     }
-    __syncthreads();
-    if (t == 0) meta[34] = flag;
   }
+  const int bad = __syncthreads_or(mx >= kBf16MaxBits);
+  if (t == 0) a.flags[slot * kTileFlags + blockIdx.y] = bad;
 }
 
 // One row's 8-value chunk halves as the prefill GEMM's x' (pair order (0,4)
@@ -317,21 +234,21 @@ __device__ __forceinline__ u32x4 xprep_chunk(const float (&v)[4], int e, bool od
 // Masked keys get weight exactly 0; tiles that a wave's rows do not see are
 // skipped by that wave.
 template <int HD>
-__global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(RowsArgs a) {
+__global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_split_kernel(RowsArgs a) {
   constexpr int DH = kDimWaves<HD>, WV = 4 * DH, NTH = 64 * WV;
   constexpr int NJ = HD / 32 / DH, NN = HD / 16 / DH;  // of one wave's dims
-  constexpr int KP = 3 * NJ * DH, VP = NN * DH;        // 1 KB pieces of 16 keys of K, of V's half
+  constexpr int KP = 3 * NJ * DH, VP = 3 * NN * DH / 2;  // 1 KB pieces of 16 keys of K, of V's half
   constexpr int KW = (KP + WV - 1) / WV, VW = VP / WV;  // and loads per wave
   constexpr int KU = KP * 64, VU = VP * 64;             // units of a buffer
   struct Smem {
     u32x4 a[KU];
     u32x4 b[KU > VU ? KU : VU];
     u32x4 c[VU];
-    int meta[kMetaInts];
-    f32x4 ex[DH > 1 ? WV : 0][2][64];  // partial scores of waves that share rows
-    float mx[DH > 1 ? WV : 0][16];
+    // partial scores of waves that share rows; before and after the tiles, one
+    // value per wave or lane
+    f32x4 ex[DH > 1 ? WV : 1][2][64];
   };
-  __shared__ Smem sm;
+  __shared__ Smem sm;  // head dim 512: all of a CU's 160 KB
   typedef __attribute__((address_space(3))) void *lds_ptr;
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int c = lane & 15, g = lane >> 4;
@@ -372,7 +289,11 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
   const int in1 = R0 + 16 * rg + 15 < nrows ? (sp.qpos0 + Rf / H + 1) / kTile - 1 : -1;
 
   const int base = sp.base(a);
-  auto tile = [&](int kt) { return a.kv + (size_t)(kt - base) * (20 * HD); };
+  auto tile = [&](int kt) { return a.kv + (size_t)(kt - base) * (24 * HD); };
+  auto flagged = [&](int kt) {
+    const int *f = a.flags + (kt - base) * kTileFlags;
+    return (f[0] | f[1]) != 0;
+  };
   auto load = [&](const u32x4 *src, u32x4 *dst, int pieces, int n) {
 #pragma unroll
     for (int i = 0; i < n; ++i) {
@@ -385,10 +306,7 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
     load(tile(kt) + sub * (6 * HD), sub ? sm.b : sm.a, KP, KW);
   };
   auto load_v = [&](int kt, int half) {
-    load(tile(kt) + 12 * HD + half * (4 * HD), half ? sm.b : sm.c, VP, VW);
-    if (half == 0)
-      __builtin_amdgcn_global_load_lds(
-          (const void *)(a.meta + (size_t)(kt - base) * kMetaInts + lane), (lds_ptr)sm.meta, 4, 0, 0);
+    load(tile(kt) + 12 * HD + half * (6 * HD), half ? sm.b : sm.c, VP, VW);
   };
   load_k(t0, 0);
   load_k(t0, 1);
@@ -396,7 +314,7 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
 
   // q of this lane's row: dims 32 j + 8 g .. + 7, as three parts
   bf16x8 qp[NJ][3];
-  bool qslow;
+  bool qslow, any_slow;  // of the block: a q beyond BF16's range; that or a flagged tile
   {
     const float4 *src = reinterpret_cast<const float4 *>(a.q + (size_t)R * HD + dh * (HD / DH) + 8 * g);
     float x[NJ][8];
@@ -414,9 +332,19 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
         const uint32_t b = __float_as_uint(x[j][i]) & 0x7fffffffu;
         mx = b > mx ? b : mx;
       }
-    qslow = __syncthreads_or(mx >= kBf16MaxBits);
+    bool f = false;
+    for (int kt = t0 + t; kt <= t1; kt += NTH) f = f || flagged(kt);
+    int *fl = reinterpret_cast<int *>(sm.ex);
+    const int slow = (__any(mx >= kBf16MaxBits) ? 1 : 0) | (__any(f) ? 2 : 0);
+    if (lane == 0) fl[w] = slow;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) split8(x[j], qp[j]);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    int all = 0;
+#pragma unroll
+    for (int i = 0; i < WV; ++i) all |= fl[i];
+    qslow = __builtin_amdgcn_readfirstlane(all) & 1;
+    any_slow = __builtin_amdgcn_readfirstlane(all) != 0;
   }
 
   float m = -1e30f, l = 0.f;  // l: this lane's keys only
@@ -424,17 +352,16 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
 #pragma unroll
   for (int n = 0; n < NN; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   for (int kt = t0; kt <= t1; ++kt) {
     const bool mine = kt >= wt0 && kt <= wt1;
-    f16x8 ph, pl;
-    float p[8], s[8], osc = 0.f;
+    bf16x8 pp[3];
+    float s[8];
     bool slow = false;
     // the scores of 16 keys over this wave's dims: the leading products in sums
     // of 128 dims.  The order of reads and products is the compiler's, and the
-    // wave goes first on its SIMD meanwhile (1500 rows over 3000 keys: 384 us
-    // with one step's pieces read ahead by scheduling groups, 375 so; for the
-    // outputs below the groups are worth 583 against 657 us at 2048 over 4096)
+    // wave goes first on its SIMD meanwhile (one step's pieces read ahead by
+    // scheduling groups cost 2% of a call of 1500 rows over 3000 keys; for the
+    // outputs below the groups are worth 670 against 721 us at 2048 over 4096)
     auto scores = [&](const u32x4 *buf, float *sc) {
       const u32x4 *kb = buf + dh * (NJ * 3 * 64) + lane;
       constexpr int NM = NJ > 4 ? NJ / 4 : 1;
@@ -492,7 +419,7 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
         }
       }
       const bool inner = kt >= in0 && kt <= in1;
-      slow = qslow || __builtin_amdgcn_readfirstlane(sm.meta[33] | sm.meta[34]) != 0;
+      if (any_slow) slow = qslow || __builtin_amdgcn_readfirstlane(flagged(kt) ? 1 : 0) != 0;
       auto key_of = [&](int i) { return kt * kTile + (i < 4 ? 4 * g + i : 12 + 4 * g + i); };
       if (slow) {
 #pragma unroll
@@ -520,28 +447,14 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
       const float mn = fmaxf(m, group_max(tm) * kLog2e);
       const float corr = __builtin_amdgcn_exp2f(m - mn);
       m = mn;
-      const f32x4 f0 = *reinterpret_cast<const f32x4 *>(&sm.meta[4 * g]);
-      const f32x4 f1 = *reinterpret_cast<const f32x4 *>(&sm.meta[16 + 4 * g]);
-      const int em = sm.meta[32];
-      float ls = 0.f, pm = 0.f, x[8];
+      float ls = 0.f, p[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         p[i] = __builtin_amdgcn_exp2f(fmaf(s[i], kLog2e, -mn));  // 0 for a masked key
         ls += p[i];
-        x[i] = p[i] * (i < 4 ? f0[i & 3] : f1[i & 3]);
-        pm = fmaxf(pm, x[i]);
       }
       l = fmaf(l, corr, ls);
-      int z = 14 - __builtin_amdgcn_frexp_expf(group_max(pm));
-      z = z < 100 ? z : 100;
-      osc = ldexpf(1.f, em - z);
-      const float zf = ldexpf(1.f, z);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float y = x[i] * zf;
-        ph[i] = (_Float16)y;
-        pl[i] = (_Float16)(y - (float)ph[i]);
-      }
+      split8(p, pp);
       if (__any(corr != 1.f)) {
 #pragma unroll
         for (int n = 0; n < NN; ++n) o[n] *= corr;
@@ -549,38 +462,35 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
     }
     auto outputs = [&](const u32x4 *buf, auto half) {
       constexpr int n0 = decltype(half)::value * (NN / 2);
-      const u32x4 *vb = buf + dh * (NN * 64) + lane;
-      f16x8 vv[NN / 2][2];
+      const u32x4 *vb = buf + dh * (NN / 2 * 3 * 64) + lane;
+      bf16x8 vv[NN / 2][3];
 #pragma unroll
-      for (int i = 0; i < NN / 2; ++i) {
-        vv[i][0] = __builtin_bit_cast(f16x8, vb[(2 * i) * 64]);
-        vv[i][1] = __builtin_bit_cast(f16x8, vb[(2 * i + 1) * 64]);
-      }
+      for (int i = 0; i < NN / 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) vv[i][q] = __builtin_bit_cast(bf16x8, vb[(3 * i + q) * 64]);
+      constexpr int kProducts[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
 #pragma unroll
       for (int i = 0; i < NN / 2; i += 2) {
-        f32x4 d[2];
+        f32x4 d[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-          d[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[i + u][1], ph, (f32x4){0.f, 0.f, 0.f, 0.f},
-                                                        0, 0, 0);
+        for (int q = 0; q < 6; ++q)
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-          d[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[i + u][0], pl, d[u], 0, 0, 0);
+          for (int u = 0; u < 2; ++u)
+            d[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv[i + u][kProducts[q][0]],
+                                                           pp[kProducts[q][1]], d[u], 0, 0, 0);
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-          d[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[i + u][0], ph, d[u], 0, 0, 0);
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) o[n0 + i + u][v] = fmaf(d[u][v], osc, o[n0 + i + u][v]);
+        for (int u = 0; u < 2; ++u) o[n0 + i + u] += d[u];
       }
       constexpr int AHEAD = 2;
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * AHEAD, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 3 * AHEAD, 0);
 #pragma unroll
       for (int i = 0; i < NN / 2; i += 2) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
-        if (i + AHEAD < NN / 2) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-        if (i > 0) __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+          if (i + AHEAD < NN / 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          if (i > 0) __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        }
       }
     };
     if (mine && !slow) outputs(sm.c, std::integral_constant<int, 0>());
@@ -592,7 +502,7 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
       for (int gg = 0; gg < 4; ++gg)
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const float pk = __shfl(p[i], 16 * gg + c, 64);
+          const float pk = __shfl((float)pp[0][i] + ((float)pp[1][i] + (float)pp[2][i]), 16 * gg + c, 64);
           const int key = kt * kTile + (i < 4 ? 4 * gg + i : 12 + 4 * gg + i);
           if (!(live && key <= rpos && key < sp.keylen && key > rlo)) continue;
           const float *vp = a.v + (size_t)key * HD + dh * (HD / DH) + 4 * g;
@@ -642,9 +552,10 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_f16_kernel(R
   mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
   if (DH > 1) {
-    if (g == 0) sm.mx[w][c] = mx;
+    float *rmx = reinterpret_cast<float *>(sm.ex);
+    if (g == 0) rmx[16 * w + c] = mx;
     __syncthreads();
-    mx = fmaxf(sm.mx[rg][c], sm.mx[rg + 4 * (DH - 1)][c]);
+    mx = fmaxf(rmx[16 * rg + c], rmx[16 * (rg + 4 * (DH - 1)) + c]);
   }
   const int e = mx > 0.f && mx <= 3.4e38f ? ilogbf(mx) - 13 : 0;
   const int qr = Rw / H, h = Rw - qr * H;
@@ -777,7 +688,7 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 struct RowsPlan {
   int tiles, tps, splits;
-  size_t kv, meta, part, total;  // floats
+  size_t kv, flags, part, total;  // floats
 };
 
 constexpr int kMaxKeys = 16384;  // launch_attention's limit
@@ -796,14 +707,17 @@ int keys_seen(int positions, int max_keylen, bool sliding, int window) {
 // least two tiles each, and no more than `avail` floats of scratch).
 // Head dim 256: as many as fill the CUs with two blocks each.
 // Head dim 512, one block per CU: the split whose blocks, dealt to the CUs in
-// launch order, end first by these measured costs in halves of a tile's 4.4 us:
-// 2 per tile, 4 per block (q's conversion, the first loads, the stores), 1 for a
-// block with no tiles (early rows have fewer than late ones, yet every block
-// needs its LDS), and with more than one split 3 for the merge and 1 per 36
-// blocks for its planes.  us per call at 8 heads by splits (* as chosen): 1000
-// rows over 1000 keys 175, 111, 88 *, 117; 700 over 2700 keys 419, 238, 175 *,
-// 247; 1500 over 1500 keys 247, 155 *, 197; 2048 over 4096 keys 623, 657, 611,
-// 580 *, 582, 626.
+// launch order, end first by these costs in halves of a tile's 5.2 us: 2 per
+// tile, 4 per block (q's conversion, the first loads, the stores), 1 for a block
+// with no tiles (early rows have fewer than late ones, yet every block needs its
+// LDS), and with more than one split 3 for the merge and 1 per 36 blocks for its
+// planes.  us per call at 8 heads (* as chosen), 1, 2, 3, 4, 5 splits, then 6 and 8:
+//   1000 rows, 1000 keys  201 124   96*  127 123  114 126
+//    700 rows, 2700 keys  493 271  196*  286 238  217 248
+//   1500 rows, 1500 keys  286 173* 222   186 183  195 208
+//   2048 rows, 4096 keys  730 766  708   671* 677  726 776
+//    300 rows,  900 keys  180 110   83    72  61   56  59*
+//   1500 rows, 3000 keys  542 430* 412   458 394  434 442
 bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int window,
                size_t avail, RowsPlan *p) {
   const int nrows = qrows * heads, blocks = cdiv(nrows, kRows);
@@ -814,8 +728,8 @@ bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int w
     return n < all ? n : all;
   };
   p->tiles = tiles_of(qrows);
-  p->kv = (size_t)p->tiles * hd * 80;
-  p->meta = (size_t)p->tiles * kMetaInts;
+  p->kv = (size_t)p->tiles * hd * 96;
+  p->flags = ((size_t)p->tiles * kTileFlags + 3) & ~size_t(3);
   const int nt = tiles_of(span < qrows ? span : qrows);
   const int slots = cus();
   // tiles of row block b (launched last to first), as the kernel counts them
@@ -829,7 +743,7 @@ bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int w
   auto fits = [&](int splits) {
     p->splits = splits;
     p->part = splits > 1 ? (size_t)splits * nrows * (hd + 2) : 0;
-    p->total = p->kv + p->meta + p->part;
+    p->total = p->kv + p->flags + p->part;
     return p->total <= avail;
   };
   auto tiles_per = [&](int splits) {
@@ -887,8 +801,8 @@ int launch_rows(const RowsArgs &a, const RowsPlan &p) {
   G4_LAUNCH_CHECK("attn_kv_split_kernel");
   const bool pad = a.xt && p.splits == 1;
   const dim3 grid(cdiv((pad ? a.Mp : a.qrows) * a.H, kRows), p.splits);
-  hipLaunchKernelGGL(attn_rows_f16_kernel<HD>, grid, dim3(256 * kDimWaves<HD>), 0, stream(), a);
-  G4_LAUNCH_CHECK("attn_rows_f16_kernel");
+  hipLaunchKernelGGL(attn_rows_split_kernel<HD>, grid, dim3(256 * kDimWaves<HD>), 0, stream(), a);
+  G4_LAUNCH_CHECK("attn_rows_split_kernel");
   if (p.splits == 1) return G4_OK;
   if (a.xt)
     hipLaunchKernelGGL((attn_rows_merge_kernel<HD, true>), dim3(a.Mp), dim3(256), 0, stream(), a);
@@ -906,10 +820,12 @@ int launch_rows(const RowsArgs &a, const RowsPlan &p) {
 // 0.75 at 256) times the rounds of such blocks over the CUs, and 10 us.  Here a
 // call costs 25 to 35 us before keys matter (three launches, q's conversion
 // and, growing with the rows, the planes of the key splits).  Measured at 8
-// heads, FP32 kernel against this one: head dim 512, 12 rows over 212 keys
-// 31.4 / 31.2 us, 362 keys 47 / 33, 80 rows over 280 keys 39 / 36, 256 rows over
-// 256 keys 35 / 39; head dim 256, 20 rows over 220 keys 21 / 23, 370 keys 27 / 24,
-// 512 rows over 512 keys 33 / 39, 700 rows over 700 keys 51 / 45.
+// heads, FP32 kernel against this one: head dim 512, 12 rows over 362 keys 47 /
+// 33 us, 5 over 290 40 / 30, 80 over 280 38 / 36, 320 over 320 42 / 40; head dim
+// 256, 20 rows over 370 keys 26 / 22, 512 over 512 33 / 39, 700 over 700 51 / 45,
+// 1000 over 1000 65 / 50.  With 4, 2 and 1 heads (2 to 1000 rows, 0 to 2500 keys
+// before them, both head dims) the calls that the rule brings here take 0.15
+// to 1 times the FP32 kernels' time, but 1.05 at 2 heads, 1000 rows, window 512.
 bool attention_rows_wins(int qrows, int heads, int hd, int max_keylen, bool sliding, int window) {
   if ((hd != 256 && hd != 512) || max_keylen > kMaxKeys) return false;
   const int nrows = qrows * heads;
@@ -942,8 +858,8 @@ int launch_attention_rows(const float *q, const float *k, const float *v, int qr
   a.xe = xe;
   a.Mp = Mp;
   a.kv = reinterpret_cast<u32x4 *>(scratch);
-  a.meta = reinterpret_cast<int *>(scratch + p.kv);
-  a.part = scratch + p.kv + p.meta;
+  a.flags = reinterpret_cast<int *>(scratch + p.kv);
+  a.part = scratch + p.kv + p.flags;
   a.ml = reinterpret_cast<float2 *>(a.part + (size_t)p.splits * qrows * heads * hd);
   a.H = heads;
   a.hd = hd;

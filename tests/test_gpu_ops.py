@@ -290,9 +290,9 @@ def test_attention_rows_over_long_caches(g4, qrows, heads, hd, keylen, tail, sli
 
 @pytest.mark.parametrize("hd", [256, 512])
 def test_attention_rows_value_rows_of_any_size(g4, hd):
-    # value rows from 1e-18 to 1e18 (each has its own exponent).  Per element the
-    # error is a few roundings of sum p |v|: 22-bit halves of p and v (3 x 2^-22)
-    # and the p of scores rounded at 2^-24 |s| with |s| < 8, about 2^-20 in all.
+    # value rows from 1e-18 to 1e18.  Per element the error is a few roundings of
+    # sum p |v| and the p of scores rounded at 2^-24 |s| with |s| < 8, about 2^-20
+    # in all.
     qrows, heads, keylen = 12, 8, 600
     q, k, v, qpos0 = rows_case(qrows, heads, hd, keylen, 0, 22, spread=18.0)
     got = run_attention(g4, q, k, v, qrows, heads, hd, keylen, qpos0, False, 0)
