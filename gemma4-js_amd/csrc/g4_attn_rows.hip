@@ -109,6 +109,7 @@ __device__ __forceinline__ float group_max(float v) {
 }
 
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kNoScore = -1e30f;  // where a row's maximum starts (the shader's masked logit)
 constexpr uint32_t kBf16MaxBits = 0x7f7f8000u;  // from here on BF16 rounds to infinity
 
 // Waves that share a row's head dim (its q and output dims), and the place of
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_split_kernel
     any_slow = __builtin_amdgcn_readfirstlane(all) != 0;
   }
 
-  float m = -1e30f, l = 0.f;  // l: this lane's keys only
+  float m = kNoScore, l = 0.f;  // l: this lane's keys only
   f32x4 o[NN];
 #pragma unroll
   for (int n = 0; n < NN; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -441,16 +442,14 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_split_kernel
       float tm = s[0];
 #pragma unroll
       for (int i = 1; i < 8; ++i) tm = fmaxf(tm, s[i]);
-      // the running maximum in units of log 2: p = 2^(s log2 e - m), one
-      // rounding of the exponent's argument.  (fmaxf drops a NaN score, whose
-      // p is NaN.)
-      const float mn = fmaxf(m, group_max(tm) * kLog2e);
-      const float corr = __builtin_amdgcn_exp2f(m - mn);
+      // (fmaxf drops a NaN score, whose p is NaN.)
+      const float mn = fmaxf(m, group_max(tm));
+      const float corr = __builtin_amdgcn_exp2f((m - mn) * kLog2e);
       m = mn;
       float ls = 0.f, p[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        p[i] = __builtin_amdgcn_exp2f(fmaf(s[i], kLog2e, -mn));  // 0 for a masked key
+        p[i] = __builtin_amdgcn_exp2f((s[i] - mn) * kLog2e);  // 0 for a masked key
         ls += p[i];
       }
       l = fmaf(l, corr, ls);
@@ -570,8 +569,8 @@ __global__ __launch_bounds__(256 * kDimWaves<HD>, 2) void attn_rows_split_kernel
   }
 }
 
-// Adds the key splits of one query row: out = sum_s 2^(m_s - M) o_s /
-// sum_s 2^(m_s - M) l_s in split order, as rows of out or as the GEMM's x'.
+// Adds the key splits of one query row: out = sum_s e^(m_s - M) o_s /
+// sum_s e^(m_s - M) l_s in split order, as rows of out or as the GEMM's x'.
 // A block is one query row (x': all heads, one exponent) or one (query row,
 // head); thread t takes 16-byte units t, t + 256, ... of it.
 template <int HD, bool X>
@@ -597,7 +596,7 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsArgs a) {
     const int nt = sp.kmax(sp.qpos0 + re / H) / kTile - sp.kmin(a, sp.qpos0 + r0 / H) / kTile + 1;
     return (nt + a.tps - 1) / a.tps;
   };
-  // weights 2^(m_s - M) and the sum of each head: 16 lanes per head
+  // weights e^(m_s - M) and the sum of each head: 16 lanes per head
   {
     const int hh = t >> 4, li = t & 15;
     const int R = qr * H + h0 + (hh < nh ? hh : 0), ns = splits(R);
@@ -614,7 +613,7 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(RowsArgs a) {
 #pragma unroll
     for (int i = 0; i < kMaxSplits / 16; ++i) {
       const int s = li + 16 * i;
-      const float e = s < ns ? __builtin_amdgcn_exp2f(ml[i].x - M) : 0.f;
+      const float e = s < ns ? __builtin_amdgcn_exp2f((ml[i].x - M) * kLog2e) : 0.f;
       if (hh < nh) wt[hh][s] = e;
       L += s < ns ? e * ml[i].y : 0.f;
     }

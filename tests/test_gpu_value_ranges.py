@@ -73,3 +73,19 @@ def test_attention_keeps_tiny_values(g4, hd):
     case[2][:, ::3] *= np.float32(1e-28)
     case[2][:, 1::3] *= np.float32(1e-33)
     assert_small_values_kept(g4, case, 2.0 ** -19)
+
+
+@pytest.mark.parametrize("hd", [256, 512])
+@pytest.mark.parametrize("top,other", [(3e38, 2.9e38), (-8e29, -9e29)])
+def test_attention_scores_at_the_ends_of_their_range(g4, hd, top, other):
+    # all weight on key 40's and 41's equal maxima, up to FP32's largest scores and
+    # down to the shader's masked logit of -1e30
+    case = attention_case(hd, 34)
+    q, k, v = case[:3]
+    q[:] = 0.0
+    q.reshape(-1, hd)[:, 0] = 1.5e19
+    k[:, 0] = other / 1.5e19
+    k[40:42, 0] = top / 1.5e19
+    got = attend(g4, *case)
+    want = np.tile(0.5 * (v[40] + v[41]), (case[3], case[4]))
+    np.testing.assert_allclose(got, want, rtol=1e-6, atol=1e-6)
