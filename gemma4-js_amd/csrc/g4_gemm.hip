@@ -1421,43 +1421,18 @@ int w4_gemm_ext(const g4_w4 *w, const void *x, bool f32x, int rows, void *y, boo
   return gemm_run(&w, 1, x, f32x, rows, &y, y_bf16, nullptr, false, &ext);
 }
 
-// Two FP32 rows of one slice, three and four always: against the GEMV of as
-// many rows, us at K x N 1536 x 6144 and 6144 x 1536 (three slices and a sum
-// launch): two rows 6.8 / 6.7 and 8.2 / 8.8, three 8.6 / 6.8 and 13.3 / 9.2,
-// four 10.0 / 7.0 and 15.7 / 9.5; K 12288: 18.5 / 11.0, 27 / 11.5, 35.8 / 11.7.
-// With BF16 x the GEMV needs half the arithmetic and keeps up to four rows.
-static bool few_rows_plan(const g4_w4 *const *w, int nw, int rows, GemmSmallPlan *p) {
-  return gemm_small_plan(w, nw, rows, false, true, p) &&
-         (rows > 2 || p->slices == 1 || w[0]->K > 8192);
-}
-
-int w4_gemm_few(const g4_w4 *w, const void *x, int rows, void *y, bool y_bf16,
-                const ExtScratch *ext, bool *taken) {
+// Plans of one slice: two to four rows need no scratch, so that their calls may
+// overlap and be recorded at any time.  Against the GEMV of as many rows, us at
+// K x N 1536 x 6144: two rows 6.8 / 6.7, three 8.6 / 6.8, four 10.0 / 7.0.  With
+// BF16 x the GEMV needs half the arithmetic and keeps up to four rows.
+int w4_gemm_few(const g4_w4 *const *w, int nw, const void *x, int rows, void *const *y,
+                bool y_bf16, bool *taken) {
   GemmSmallPlan p;
-  *taken = false;
-  if (!few_rows_plan(&w, 1, rows, &p)) return G4_OK;
-  const size_t need = part_bytes(&w, 1, rows, p.slices);
-  void *ws = nullptr;
-  // the GEMV needs no scratch: it stays where none can be had
-  if (ext) {
-    if (need > ext->bytes) return G4_OK;
-    ws = ext->mem;
-  } else if (need > 0) {
-    if (encoding() && g_ws.bytes < need) return G4_OK;
-    if (int rc = g_ws.get(need, &ws, "g4_w4_linear (few rows)")) return rc;
-  }
-  *taken = true;
-  float *part = static_cast<float *>(ws);
-  const size_t pstride = splitk_pstride(rows, w->N);
-  if (int rc = launch_gemm_small(p, &w, 1, x, true, nullptr, nullptr, 0, rows, &y, y_bf16, part,
-                                 pstride, false))
-    return rc;
-  return p.slices > 1 ? launch_splitk_sum(part, p.slices, &w, 1, rows, &y, y_bf16) : G4_OK;
-}
-
-bool w4_gemm_few_joint(const g4_w4 *const *w, int nw, int rows) {
-  GemmSmallPlan p;
-  return nw > 1 && rows > 1 && rows <= kMaxGemvRows && few_rows_plan(w, nw, rows, &p);
+  *taken = rows > 1 && rows <= kMaxGemvRows && gemm_small_plan(w, nw, rows, false, true, &p) &&
+           p.slices == 1;
+  return *taken ? launch_gemm_small(p, w, nw, x, true, nullptr, nullptr, 0, rows, y, y_bf16, nullptr,
+                                    0, false)
+                : G4_OK;
 }
 
 int w4_gemm_glu(const g4_w4 *gate, const g4_w4 *up, const float *x, int rows, float *act) {

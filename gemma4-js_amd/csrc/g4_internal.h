@@ -163,11 +163,10 @@ struct ExtScratch {
 int w4_gemm_ext(const g4_w4 *w, const void *x, bool f32x, int rows, void *y, bool y_bf16,
                 const ExtScratch &ext);
 // 2 to kMaxGemvRows FP32 rows where the few-row matrix-core kernel beats the
-// GEMV (*taken; else nothing is launched), and whether it takes several weights
-// of one in_dim in one launch (through w4_gemm_multi).
-int w4_gemm_few(const g4_w4 *w, const void *x, int rows, void *y, bool y_bf16,
-                const ExtScratch *ext, bool *taken);
-bool w4_gemm_few_joint(const g4_w4 *const *w, int nw, int rows);
+// GEMV and needs no scratch (*taken; else nothing is launched), for nw weights
+// of one in_dim in one launch.
+int w4_gemm_few(const g4_w4 *const *w, int nw, const void *x, int rows, void *const *y,
+                bool y_bf16, bool *taken);
 // g4_w4_linear's argument checks and dispatch; with ext set, the GEMM path
 // uses that scratch (the GEMV paths use none).
 int w4_linear_impl(const g4_w4 *w, const void *x, int x_dtype, int rows, void *y, int y_dtype,

@@ -1204,7 +1204,7 @@ int w4_linear_impl(const g4_w4 *w, const void *x, int x_dtype, int rows, void *y
                 : launch_gemv1<false>(w, x, y, y_dtype == G4_BF16);
   if (f32x && rows > 1 && rows <= kMaxGemvRows && gemv_fits) {
     bool taken;
-    const int rc2 = w4_gemm_few(w, x, rows, y, y_dtype == G4_BF16, ext, &taken);
+    const int rc2 = w4_gemm_few(&w, 1, x, rows, &y, y_dtype == G4_BF16, &taken);
     if (rc2 || taken) return rc2;
   }
   if (rows > kMaxGemvRows || !gemv_fits)
@@ -1243,7 +1243,7 @@ G4_API int g4_w4_linear_multi(const g4_w4 *const *w, int n, const void *x, int x
       return fail(G4_E_ARG, "g4_w4_linear_multi: weight %d has in_dim %d, weight 0 has %d", i,
                   w[i]->K, w[0]->K);
   }
-  const bool few = x_dtype == G4_F32 && w4_gemm_few_joint(w, n, rows);
+  const bool few = n > 1 && x_dtype == G4_F32 && rows > 1 && rows <= kMaxGemvRows;
   if (n == 1 || (rows > 1 && rows <= kMaxGemvRows && !few) ||
       (rows == 1 && !has_gemv1_plan(w[0]->G, x_dtype == G4_F32))) {
     for (int i = 0; i < n; ++i)
@@ -1264,6 +1264,13 @@ G4_API int g4_w4_linear_multi(const g4_w4 *const *w, int n, const void *x, int x
   for (int i = 0; i < n; ++i)
     if ((rc = check_device_range(y[i], (size_t)rows * w[i]->N * ye, "g4_w4_linear_multi y")))
       return rc;
+  if (few) {
+    bool taken;
+    if ((rc = w4_gemm_few(w, n, x, rows, y, y_dtype == G4_BF16, &taken))) return rc;
+    for (int i = 0; i < n && !taken; ++i)
+      if ((rc = g4_w4_linear(w[i], x, x_dtype, rows, y[i], y_dtype))) return rc;
+    return ok();
+  }
   // more than kMaxGemvRows, or an in_dim beyond the GEMV's LDS staging: one
   // x pre-pass, one GEMM launch when it fills
   if (rows > 1 || gemv_lds_per_row(w[0]->K, f32x) > kGemvLdsBudget) {

@@ -183,7 +183,9 @@ int g4_w4_linear_noalloc(const g4_w4 *w, const void *x, int x_dtype, int rows,
  * 1 <= n <= 3, every W[i] of the same in_dim, outputs as g4_w4_linear's.
  * One activation row runs the n GEMVs as one launch; more than 4 rows share
  * one activation pre-pass and, when the weights' tiles fill the GPU, one GEMM
- * launch; 2-4 rows take g4_w4_linear per weight.  The outputs must not
+ * launch; 2-4 rows share one launch where it needs no scratch (FP32 x,
+ * in_dim <= 2048, tiles that fit the GPU in one round), else they take
+ * g4_w4_linear per weight, with the same results.  The outputs must not
  * overlap x or each other. */
 int g4_w4_linear_multi(const g4_w4 *const *w, int n, const void *x, int x_dtype,
                        int rows, void *const *y, int y_dtype);
