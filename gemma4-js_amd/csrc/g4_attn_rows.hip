@@ -825,8 +825,9 @@ int launch_rows(const RowsArgs &a, const RowsPlan &p) {
 // 1000 over 1000 65 / 50.  With 4, 2 and 1 heads (2 to 1000 rows, 0 to 2500 keys
 // before them, both head dims) the calls that the rule brings here take 0.15
 // to 1 times the FP32 kernels' time, but 1.05 at 2 heads, 1000 rows, window 512.
+// One row has kernels of its own.
 bool attention_rows_wins(int qrows, int heads, int hd, int max_keylen, bool sliding, int window) {
-  if ((hd != 256 && hd != 512) || max_keylen > kMaxKeys) return false;
+  if (qrows < 2 || (hd != 256 && hd != 512) || max_keylen > kMaxKeys) return false;
   const int nrows = qrows * heads;
   const int keys = keys_seen(cdiv(16, heads) + 1, max_keylen, sliding, window);
   const int steps = cdiv(keys, 16) * cdiv(nrows, 16 * cus());

@@ -47,3 +47,24 @@ again = [y.download(np.uint32) for y in ys]
 assert all(np.array_equal(a, b) for a, b in zip(first, again))
 assert np.array_equal(first[0], first[1]) and np.array_equal(first[0], first[2])
 """ % (k, rows))
+
+
+def test_one_row_attention_holds_its_partials_only():
+    # one row over 16384 keys at head dim 512: 1024 splits of 8 x 514 floats, 17 MB
+    out = fresh("""
+hip = ctypes.CDLL("libamdhip64.so")
+def free():
+    a, b = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+    return a.value
+keys, hd = 16384, 512
+q, y = g4.Buffer(8 * hd * 4), g4.Buffer(8 * hd * 4)
+k, v = g4.Buffer(keys * hd * 4), g4.Buffer(keys * hd * 4)
+g4.attention(q, k, v, 1, 8, hd, 64, 63, False, 0, y)
+g4.sync()
+before = free()
+g4.attention(q, k, v, 1, 8, hd, keys, keys - 1, False, 0, y)
+g4.sync()
+print(before - free())
+""")
+    assert int(out) < 24 << 20, out
