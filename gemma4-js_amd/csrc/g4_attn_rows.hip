@@ -31,7 +31,9 @@
 // call takes 82% of its time, without the score products 67%, without the output
 // products 78%, with softmax and barriers alone 25%.  (v and p as two FP16 parts,
 // three products, took 568 us there and 365 over 3000 keys.)
+#include <limits.h>
 #include <math.h>
+#include <string.h>
 
 #include <type_traits>
 
@@ -694,13 +696,22 @@ constexpr int kMaxKeys = 16384;  // launch_attention's limit
 constexpr int kRing = 2048;
 static_assert(2 * (kMaxKeys / kTile + 1) + 4 < kRing, "a block's time fits the ring");
 
-int cus() { return cu_count() > 0 ? cu_count() : 256; }
+constexpr int kMaxCus = 512;
+int cus() {
+  const int n = cu_count();
+  return n <= 0 ? 256 : n < kMaxCus ? n : kMaxCus;
+}
 
 // Most keys that the rows of `positions` consecutive positions see.
 int keys_seen(int positions, int max_keylen, bool sliding, int window) {
   const long n = (long)window - 1 + positions;
   return sliding && n < max_keylen ? (int)n : max_keylen;
 }
+
+// What a plan depends on besides the scratch.
+struct RowsKey {
+  int qrows, heads, hd, max_keylen, sliding, window, cus;
+};
 
 // Key tiles of the call, and the split of a row block's tiles over blocks (at
 // least two tiles each, and no more than `avail` floats of scratch).
@@ -717,8 +728,10 @@ int keys_seen(int positions, int max_keylen, bool sliding, int window) {
 //   2048 rows, 4096 keys  730 766  708   671* 677  726 776
 //    300 rows,  900 keys  180 110   83    72  61   56  59*
 //   1500 rows, 3000 keys  542 430* 412   458 394  434 442
-bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int window,
-               size_t avail, RowsPlan *p) {
+bool find_plan(const RowsKey &key, size_t avail, RowsPlan *p) {
+  const int qrows = key.qrows, heads = key.heads, hd = key.hd, max_keylen = key.max_keylen;
+  const int window = key.window;
+  const bool sliding = key.sliding != 0;
   const int nrows = qrows * heads, blocks = cdiv(nrows, kRows);
   const int span = cdiv(kRows, heads) + 1;  // positions of a block's rows
   const int all = cdiv(max_keylen, kTile);
@@ -730,7 +743,7 @@ bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int w
   p->kv = (size_t)p->tiles * hd * 96;
   p->flags = ((size_t)p->tiles * kTileFlags + 3) & ~size_t(3);
   const int nt = tiles_of(span < qrows ? span : qrows);
-  const int slots = cus();
+  const int slots = key.cus;
   // tiles of row block b (launched last to first), as the kernel counts them
   const int qpos0 = max_keylen - qrows;
   auto block_tiles = [&](int b) {
@@ -758,10 +771,16 @@ bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int w
     }
     return false;
   }
+  if (blocks > 2 * slots) {  // more than the limit below with any split
+    p->tps = nt;
+    return fits(1);
+  }
+  int tiles[2 * kMaxCus];
+  for (int b = 0; b < blocks; ++b) tiles[b] = block_tiles(b);
   // CUs that become free at each time, from `now` on (a block takes less than a
   // turn of the ring: see kMaxKeys)
   int free_at[kRing];
-  long best = -1;
+  long best = LONG_MAX;
   int best_splits = 0, best_tps = 0, last_tps = 0;
   for (int want = 1; want <= kMaxSplits; want += want < 6 ? 1 : want / 3) {
     const int tps = tiles_per(want), splits = cdiv(nt, tps);
@@ -771,27 +790,45 @@ bool rows_plan(int qrows, int heads, int hd, int max_keylen, bool sliding, int w
     if (!fits(splits)) continue;
     for (int &f : free_at) f = 0;
     free_at[0] = slots;
-    long end = 0, used = 0, now = 0;
-    for (int y = 0; y < splits; ++y)
-      for (int b = blocks - 1; b >= 0; --b) {
-        int t = block_tiles(b) - y * tps;
+    long end = 0, used = 0;
+    unsigned now = 0;
+    for (int y = 0; y < splits && end < best; ++y)
+      for (int b = blocks - 1; b >= 0 && end < best; --b) {
+        int t = tiles[b] - y * tps;
         t = t < tps ? t : tps;
         const int len = t > 0 ? 2 * t + 4 : 1;
         used += t > 0;
         while (free_at[now % kRing] == 0) ++now;
         --free_at[now % kRing];
         ++free_at[(now + len) % kRing];
-        if (now + len > end) end = now + len;
+        if ((long)now + len > end) end = (long)now + len;
       }
     if (splits > 1) end += 3 + used / 36;
-    if (best < 0 || end < best) {
+    if (end < best) {
       best = end;
       best_splits = splits;
       best_tps = tps;
     }
   }
   p->tps = best_tps;
-  return best >= 0 && fits(best_splits);
+  return best_splits > 0 && fits(best_splits);
+}
+
+// The plan for at most `avail` floats.  At head dim 512 finding it takes 5 to 15 us
+// of host time, more than a call's launches, so the one for any scratch is kept
+// per thread for the last key (a call asks for its scratch and then launches, an
+// engine's layers follow each other); where it fits, it is also the best that
+// fits.
+bool rows_plan(const RowsKey &key, size_t avail, RowsPlan *p) {
+  if (key.hd <= 256) return find_plan(key, avail, p);
+  static thread_local RowsKey last{};
+  static thread_local RowsPlan plan{};
+  if (memcmp(&last, &key, sizeof(key)) != 0) {
+    find_plan(key, ~size_t(0), &plan);
+    last = key;
+  }
+  *p = plan;
+  return plan.total <= avail || find_plan(key, avail, p);
 }
 
 template <int HD>
@@ -838,7 +875,7 @@ size_t attention_rows_floats(int qrows, int heads, int hd, int max_keylen, bool 
                              int window) {
   RowsPlan p{};
   if (!attention_rows_wins(qrows, heads, hd, max_keylen, sliding, window)) return 0;
-  rows_plan(qrows, heads, hd, max_keylen, sliding, window, ~size_t(0), &p);
+  rows_plan({qrows, heads, hd, max_keylen, sliding, window, cus()}, ~size_t(0), &p);
   return p.total;
 }
 
@@ -848,7 +885,7 @@ int launch_attention_rows(const float *q, const float *k, const float *v, int qr
                           float *out, void *xt, int *xe, int Mp, bool *taken) {
   RowsPlan p{};
   *taken = false;
-  if (!rows_plan(qrows, heads, hd, max_keylen, sliding, window, scratch_floats, &p)) return G4_OK;
+  if (!rows_plan({qrows, heads, hd, max_keylen, sliding, window, cus()}, scratch_floats, &p)) return G4_OK;
   RowsArgs a{};
   a.q = q;
   a.k = k;
