@@ -98,7 +98,12 @@ void *g4_stream(void);
  * with G4_E_STATE while an encoder is open.  Unlike a WebGPU command buffer,
  * a finished recording may be submitted any number of times, also after
  * later calls made the library's internal scratch grow: scratch outgrown
- * while a recording exists is kept until the last recording is freed. */
+ * while a recording exists is kept until the last recording is freed.
+ * Recording cannot make scratch grow.  A call gives the eager call's bits in a
+ * recording once one eager call of its arguments' sizes has been made; without
+ * one it fails with G4_E_STATE or, where the scratch that is there holds a form
+ * that needs less (g4_attention of several rows, g4_w4_linear_multi), records
+ * that form: as accurate, slower, and with roundings of its own. */
 typedef struct g4_cmdbuf g4_cmdbuf;
 int g4_encoder_begin(void);
 int g4_encoder_finish(g4_cmdbuf **out);
