@@ -1358,8 +1358,11 @@ int launch_norm_rope(const float *x, int rows, int heads, int hd, int pos0, cons
     return fail(G4_E_ARG, "norm_rope: %d planes (1..%d)", parts, kNormRopeMaxParts);
   if (hd > 2 * kBlock)
     return fail(G4_E_ARG, "norm_rope: head_dim %d (at most %d)", hd, 2 * kBlock);
-  // many heads of 256 or 512: four to a wave where that leaves a wave per SIMD
-  if (heads % 4 == 0 && (hd == 256 || hd == 512) && rows * heads >= 2048 && parts <= 4) {
+  // many heads of 256 or 512: four to a wave, which takes longer by itself and pays
+  // where a block per head needs a second round of blocks (us per call, block per
+  // head / four to a wave: head dim 256, 1024 heads in all 3.0 / 3.9, 2048 3.99 /
+  // 4.05, 3112 5.3 / 4.2, 8000 9.8 / 5.3; 512, 2048 4.39 / 4.45, 3112 5.9 / 4.7)
+  if (heads % 4 == 0 && (hd == 256 || hd == 512) && rows * heads > 2048 && parts <= 4) {
     void (*k4)(const float *, int, size_t, int, int, int, const int *, const float *, int, float,
                float, float *, int) = nullptr;
     switch (parts) {
